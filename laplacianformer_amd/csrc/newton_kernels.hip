@@ -23,6 +23,7 @@
 #include "lf_common.h"
 #include "lf_internal.h"
 #include "mix_common.h"
+#include "newton_split.h"
 
 namespace lfamd {
 
@@ -218,16 +219,6 @@ __device__ __forceinline__ float sum_rows4(float x) {
   return c + d;
 }
 
-// P = f32(mat) + 0.01 I on the live n x n block (the slot's padding is left as is).
-template <typename T, int NP, int WPR>
-__device__ __forceinline__ void load_P(float* __restrict__ Ps, const T* __restrict__ M, int n) {
-  using L = NsLayout<NP, WPR>;
-  for (int e = threadIdx.x; e < n * n; e += L::THREADS) {
-    const int i = e / n, j = e - i * n;
-    Ps[i * L::LS + j] = to_acc(M[e]) + (i == j ? 0.01f : 0.f);
-  }
-}
-
 // P = f32(mat) + 0.01 I on the live n x n block and zero on the rest of the
 // NP x NP slot, in one pass (each slot element written once, no zero fill
 // and barrier ahead of it).
@@ -275,16 +266,16 @@ __device__ __forceinline__ float compute_alpha(const float* __restrict__ Ps, int
 // one-live-row path with two or four waves per strip.
 template <int NP, int WPR, int KL> constexpr bool fwd_va() { return KL == 1 && WPR >= 2; }
 
-// PV_FIRST: V <- 2V - V(PV) (the reference's order for n <= 112), P held in
-// registers as this wave's A operand after the set-up, so the LDS holds V and
-// T = PV only. Otherwise V <- 2V - (VP)V (its order for n = 128): LDS holds V
-// and P, P is overwritten by W = VP and reloaded each iteration.
-template <typename T, int NP, bool PV_FIRST, int WPR, int KL>
+// V <- 2V - V(PV) (the reference's order for n <= 112) on the fp32 matrix cores, P
+// held in registers as this wave's A operand after the set-up, so the LDS holds V
+// and T = PV only. For n <= 16, and fp32 n = 49 where P is not symmetric; the other
+// sizes run on the kernels of newton_split.h.
+template <typename T, int NP, int WPR, int KL>
 __device__ __forceinline__ void newton_fwd_body(const T* __restrict__ mat, T* __restrict__ out, int n, int iters) {
   using L = NsLayout<NP, WPR>;
   extern __shared__ __align__(16) float nsm[];
   __shared__ float red[16];
-  float* Ps = nsm;                 // P; then T = PV (PV_FIRST) or W = VP
+  float* Ps = nsm;                 // P; then T = PV
   float* Vs = nsm + L::ELEMS;      // V
   // With KL = 1 the last strip's waves (one live row, on the VALU) are the
   // workgroup's first hardware waves: a SIMD issues its oldest waves first, and
@@ -323,7 +314,7 @@ __device__ __forceinline__ void newton_fwd_body(const T* __restrict__ mat, T* __
   // row r1 of P: every lane takes its k set of that row.
   constexpr int r1 = NP - 16;
   const bool rowv = KL == 1 && wave / WPR == L::NT - 1;
-  float pa[PV_FIRST ? L::NT : 1][4];
+  float pa[L::NT][4];
   auto load_pa = [&]() {  // A operand of T = P V
     const int i = rowv ? r1 : 16 * (wave / WPR) + (lane & 15), kq = 4 * (lane >> 4);
 #pragma unroll
@@ -334,7 +325,7 @@ __device__ __forceinline__ void newton_fwd_body(const T* __restrict__ mat, T* __
   };
   // Small slots: read ahead of alpha's reduction (larger ones would hold more
   // registers across it than their occupancy allows).
-  if constexpr (PV_FIRST && KEEP) load_pa();
+  if constexpr (KEEP) load_pa();
   const float alpha = compute_alpha<NP, WPR>(Ps, n, red);
   if constexpr (KEEP) {
 #pragma unroll
@@ -345,109 +336,103 @@ __device__ __forceinline__ void newton_fwd_body(const T* __restrict__ mat, T* __
   } else {
     for (int e = threadIdx.x; e < L::ELEMS; e += L::THREADS) Vs[e] = Ps[e] * alpha;
   }
-  if constexpr (PV_FIRST && !KEEP) load_pa();
+  if constexpr (!KEEP) load_pa();
 
   v4f acc[L::TW];
-  if constexpr (PV_FIRST) {
-    __syncthreads();  // P fully read (registers) and V0 written before slot P becomes T
-    float* Ts = Ps;
-    const int t0v = (wave % WPR) * L::TW, li = lane & 15, lk = lane >> 4;
-    // VA (one live row, two or four waves per strip): U = V T takes its A operand (the
-    // strip's V rows; row r1 on the row waves) from registers loaded while T is
-    // computed, so no wave reads V from LDS after T is complete and the update
-    // needs no barrier ahead of it.
-    constexpr bool VA = fwd_va<NP, WPR, KL>();
-    float va[L::NT][4];
-    auto load_va = [&]() {
-      const int i = rowv ? r1 : 16 * (wave / WPR) + li;
+  __syncthreads();  // P fully read (registers) and V0 written before slot P becomes T
+  float* Ts = Ps;
+  const int t0v = (wave % WPR) * L::TW, li = lane & 15, lk = lane >> 4;
+  // VA (one live row, two or four waves per strip): U = V T takes its A operand (the
+  // strip's V rows; row r1 on the row waves) from registers loaded while T is
+  // computed, so no wave reads V from LDS after T is complete and the update
+  // needs no barrier ahead of it.
+  constexpr bool VA = fwd_va<NP, WPR, KL>();
+  float va[L::NT][4];
+  auto load_va = [&]() {
+    const int i = rowv ? r1 : 16 * (wave / WPR) + li;
 #pragma unroll
-      for (int kb = 0; kb < L::NT; ++kb) {
-        const float4 v = *reinterpret_cast<const float4*>(&Vs[i * L::LS + 16 * kb + 4 * lk]);
-        va[kb][0] = v.x; va[kb][1] = v.y; va[kb][2] = v.z; va[kb][3] = v.w;
-      }
-    };
-    for (int it = 0; it < iters; ++it) {
-      if (rowv) {
-#pragma unroll
-        for (int t = 0; t < L::TW; ++t) {  // T[r1][j] = sum_k P[r1][k] V[k][j]
-          const int j = 16 * (t0v + t) + li;
-          float sum = 0.f;
-#pragma unroll
-          for (int kb = 0; kb < L::NT; ++kb)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              if (kb + 1 < L::NT || q < KL) sum += pa[kb][q] * Vs[(16 * kb + 4 * lk + q) * L::LS + j];
-          sum = sum_rows4(sum);
-          if (lk == 0) Ts[j * L::LS + r1] = sum;
-        }
-        if constexpr (VA) load_va();
-      } else {
-        mfma_rowstrip_areg<NP, WPR, KL>(pa, Vs, wave, lane, acc);       // T = P V
-        if constexpr (VA) load_va();  // behind T's operand reads, ahead of its barrier
-        store_strip_t<NP, WPR>(Ts, wave, lane, acc);                     // slot T holds T^T
-      }
-      __syncthreads();
-      float u[L::TW];
-      if (rowv) {
-#pragma unroll
-        for (int t = 0; t < L::TW; ++t) {  // U[r1][j] = sum_k V[r1][k] T[k][j], T[k][j] = Ts[j][k]
-          const int j = 16 * (t0v + t) + li;
-          float sum = 0.f;
-#pragma unroll
-          for (int kb = 0; kb < L::NT; ++kb) {
-            float vr[4];
-            if constexpr (VA) {
-#pragma unroll
-              for (int q = 0; q < 4; ++q) vr[q] = va[kb][q];
-            } else {
-              const float4 vv = *reinterpret_cast<const float4*>(&Vs[r1 * L::LS + 16 * kb + 4 * lk]);
-              vr[0] = vv.x; vr[1] = vv.y; vr[2] = vv.z; vr[3] = vv.w;
-            }
-            const float4 tt = *reinterpret_cast<const float4*>(&Ts[j * L::LS + 16 * kb + 4 * lk]);
-            const float ta[4] = {tt.x, tt.y, tt.z, tt.w};
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              if (kb + 1 < L::NT || q < KL) sum += vr[q] * ta[q];
-          }
-          u[t] = sum_rows4(sum);
-        }
-      } else if constexpr (VA) {
-        mfma_rowstrip_areg<NP, WPR, KL, true>(va, Ts, wave, lane, acc);    // U = V T
-      } else {
-        mfma_rowstrip<NP, WPR, false, true, KL>(Vs, Ts, wave, lane, acc);  // U = V T (own V rows only)
-      }
-      // With WPR > 1 the waves of a strip read all of its V rows and each then
-      // updates part of them: every read first (done before T was complete with VA).
-      if constexpr (WPR > 1 && !VA) __syncthreads();
-      if (rowv) {
-        if (lk == 0)
-#pragma unroll
-          for (int t = 0; t < L::TW; ++t) {
-            float* p = &Vs[r1 * L::LS + 16 * (t0v + t) + li];
-            *p = 2.0f * (*p) - u[t];
-          }
-      } else {
-        update_strip<NP, WPR>(Vs, wave, lane, acc);                    // V = 2V - U
-      }
-      __syncthreads();
+    for (int kb = 0; kb < L::NT; ++kb) {
+      const float4 v = *reinterpret_cast<const float4*>(&Vs[i * L::LS + 16 * kb + 4 * lk]);
+      va[kb][0] = v.x; va[kb][1] = v.y; va[kb][2] = v.z; va[kb][3] = v.w;
     }
-  } else {
+  };
+  for (int it = 0; it < iters; ++it) {
+    if (rowv) {
+#pragma unroll
+      for (int t = 0; t < L::TW; ++t) {  // T[r1][j] = sum_k P[r1][k] V[k][j]
+        const int j = 16 * (t0v + t) + li;
+        float sum = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < L::NT; ++kb)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (kb + 1 < L::NT || q < KL) sum += pa[kb][q] * Vs[(16 * kb + 4 * lk + q) * L::LS + j];
+        sum = sum_rows4(sum);
+        if (lk == 0) Ts[j * L::LS + r1] = sum;
+      }
+      if constexpr (VA) load_va();
+    } else {
+      mfma_rowstrip_areg<NP, WPR, KL>(pa, Vs, wave, lane, acc);       // T = P V
+      if constexpr (VA) load_va();  // behind T's operand reads, ahead of its barrier
+      store_strip_t<NP, WPR>(Ts, wave, lane, acc);                     // slot T holds T^T
+    }
     __syncthreads();
-    for (int it = 0; it < iters; ++it) {
-      mfma_rowstrip<NP, WPR, false, false>(Vs, Ps, wave, lane, acc);  // W = V P
-      __syncthreads();                                                 // P reads done
-      store_strip<NP, WPR>(Ps, wave, lane, acc);
-      __syncthreads();
-      mfma_rowstrip<NP, WPR, false, false>(Ps, Vs, wave, lane, acc);  // U = W V
-      __syncthreads();                                                 // V reads done
-      update_strip<NP, WPR>(Vs, wave, lane, acc);
-      if (it + 1 < iters) load_P<T, NP, WPR>(Ps, Mg, n);               // padding of slot P is still zero
-      __syncthreads();
+    float u[L::TW];
+    if (rowv) {
+#pragma unroll
+      for (int t = 0; t < L::TW; ++t) {  // U[r1][j] = sum_k V[r1][k] T[k][j], T[k][j] = Ts[j][k]
+        const int j = 16 * (t0v + t) + li;
+        float sum = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < L::NT; ++kb) {
+          float vr[4];
+          if constexpr (VA) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) vr[q] = va[kb][q];
+          } else {
+            const float4 vv = *reinterpret_cast<const float4*>(&Vs[r1 * L::LS + 16 * kb + 4 * lk]);
+            vr[0] = vv.x; vr[1] = vv.y; vr[2] = vv.z; vr[3] = vv.w;
+          }
+          const float4 tt = *reinterpret_cast<const float4*>(&Ts[j * L::LS + 16 * kb + 4 * lk]);
+          const float ta[4] = {tt.x, tt.y, tt.z, tt.w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (kb + 1 < L::NT || q < KL) sum += vr[q] * ta[q];
+        }
+        u[t] = sum_rows4(sum);
+      }
+    } else if constexpr (VA) {
+      mfma_rowstrip_areg<NP, WPR, KL, true>(va, Ts, wave, lane, acc);    // U = V T
+    } else {
+      mfma_rowstrip<NP, WPR, false, true, KL>(Vs, Ts, wave, lane, acc);  // U = V T (own V rows only)
     }
+    // With WPR > 1 the waves of a strip read all of its V rows and each then
+    // updates part of them: every read first (done before T was complete with VA).
+    if constexpr (WPR > 1 && !VA) __syncthreads();
+    if (rowv) {
+      if (lk == 0)
+#pragma unroll
+        for (int t = 0; t < L::TW; ++t) {
+          float* p = &Vs[r1 * L::LS + 16 * (t0v + t) + li];
+          *p = 2.0f * (*p) - u[t];
+        }
+    } else {
+      update_strip<NP, WPR>(Vs, wave, lane, acc);                    // V = 2V - U
+    }
+    __syncthreads();
   }
   // Row i by wave i mod NW, columns by lane: no division by the runtime n.
   for (int i = hw; i < n; i += L::NW)
     for (int j = lane; j < n; j += 64) Og[i * n + j] = from_acc<T>(Vs[i * L::LS + j]);
+}
+
+template <typename T, int NT>
+__global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2)))
+newton_fwd_chain_kernel(const T* __restrict__ mat, T* __restrict__ out, int n, int iters) {
+  extern __shared__ __align__(16) unsigned char chain_sm[];
+  __shared__ float red[NT];
+  const size_t off = (size_t)blockIdx.x * n * n;
+  newton_fwd_chain_body<T, NT>(mat + off, out + off, n, iters, chain_sm, red);
 }
 
 // One 16 x 16 tile of X Y (X's 16 rows in registers as in mfma_rowstrip_areg,
@@ -523,7 +508,7 @@ __device__ __forceinline__ void newton_fwd_sym_body(const float* __restrict__ ma
     if (j > i && Ps[i * L::LS + j] != Ps[j * L::LS + i]) asym = 1;
   }
   if (__syncthreads_or(asym)) {  // not symmetric: the general iteration
-    newton_fwd_body<float, NP, true, WPR, 1>(mat, out, n, iters);
+    newton_fwd_body<float, NP, WPR, 1>(mat, out, n, iters);
     return;
   }
   constexpr int r1 = NP - 16;  // the last strip's live row (48)
@@ -650,10 +635,10 @@ newton_fwd_sym_kernel(const float* __restrict__ mat, float* __restrict__ out, in
   newton_fwd_sym_body<NW>(mat, out, n, iters);
 }
 
-template <typename T, int NP, bool PV_FIRST, int WPR = 1, int KL = 4>
-__global__ void __launch_bounds__(NP * 4 * WPR)
+template <typename T, int NP>
+__global__ void __launch_bounds__(NP * 4)
 newton_fwd_kernel(const T* __restrict__ mat, T* __restrict__ out, int n, int iters) {
-  newton_fwd_body<T, NP, PV_FIRST, WPR, KL>(mat, out, n, iters);
+  newton_fwd_body<T, NP, 1, 4>(mat, out, n, iters);
 }
 
 // ---------------------------------------------------------------------------
@@ -705,8 +690,8 @@ __device__ __forceinline__ void store_tiles(float* __restrict__ dst, int wave, i
 }
 
 // The landmark forward in two launches. First, workgroups [0, bh) run
-// NewtonInverse on the bh landmark matrices (newton_fwd_body, writing the
-// inverse) and workgroups [bh, bh (1 + per)) the tall product's partials of
+// NewtonInverse on the bh landmark matrices (the bodies that lfamd_newton_forward
+// runs below two matrices per CU, writing the inverse) and workgroups [bh, bh (1 + per)) the tall product's partials of
 // K_km^T V (tall_t_bf16_body, per workgroups per slice): the two sets share
 // nothing, so the memory-bound tall product runs on the CUs that the
 // latency-bound iterations leave free. Then landmark_kv_w_kernel sums the
@@ -721,8 +706,12 @@ newton_fwd_tall_kernel(const float* __restrict__ kmm, float* __restrict__ inv, i
   if ((int)blockIdx.x < bh) {
     if constexpr (KL == 1 && NP == 64)
       newton_fwd_sym_body<8>(kmm, inv, n, iters);
-    else
-      newton_fwd_body<float, NP, true, 2, KL>(kmm, inv, n, iters);
+    else if (threadIdx.x < 64 * (NP / 16)) {  // (the other waves leave: barriers count the live ones)
+      __shared__ float red[NP / 16];
+      extern __shared__ __align__(16) float nsm[];
+      const size_t off = (size_t)blockIdx.x * n * n;
+      newton_fwd_chain_body<float, NP / 16>(kmm + off, inv + off, n, iters, reinterpret_cast<unsigned char*>(nsm), red);
+    }
   } else {
     extern __shared__ __align__(16) float nsm[];
     const int t = (int)blockIdx.x - bh;
@@ -1575,40 +1564,40 @@ template <int NP> constexpr int pick_wpr() {
 // instantiations whose last k block runs one MFMA step of four.
 template <typename T, int NP> constexpr bool has_kl1() { return std::is_same<T, float>::value && NP >= 32 && NP < 128; }
 
-template <typename T, int NP, int WPR>
-int fwd_np_w(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
-  // fp32 n = 49: the symmetric iteration when P is symmetric (the kernel checks; else the general one).
-  if constexpr (std::is_same<T, float>::value && NP == 64) {
-    if (n == NP - 15) {
-      auto k = newton_fwd_sym_kernel<WPR * 4>;
-      int s = set_lds(k, fwd_lds<NP>());
-      if (s) return s;
-      hipLaunchKernelGGL(k, dim3((unsigned)bh), dim3(NP * 4 * WPR), fwd_lds<NP>(), st, m, o, n, iters);
-      return check_launch("newton forward");
-    }
-  }
-  // The reference's association order per bucket: V(PV) below 128, (VP)V at 128.
-  if constexpr (has_kl1<T, NP>()) {
-    if (n == NP - 15) {
-      auto k = newton_fwd_kernel<T, NP, true, WPR, 1>;
-      int s = set_lds(k, fwd_lds<NP>());
-      if (s) return s;
-      hipLaunchKernelGGL(k, dim3((unsigned)bh), dim3(NP * 4 * WPR), fwd_lds<NP>(), st, m, o, n, iters);
-      return check_launch("newton forward");
-    }
-  }
-  if (NP < 128) {
-    auto k = newton_fwd_kernel<T, NP, true, WPR>;
-    int s = set_lds(k, fwd_lds<NP>());
-    if (s) return s;
-    hipLaunchKernelGGL(k, dim3((unsigned)bh), dim3(NP * 4 * WPR), fwd_lds<NP>(), st, m, o, n, iters);
-  } else {
-    auto k = newton_fwd_kernel<T, NP, false, WPR>;
-    int s = set_lds(k, fwd_lds<NP>());
-    if (s) return s;
-    hipLaunchKernelGGL(k, dim3((unsigned)bh), dim3(NP * 4 * WPR), fwd_lds<NP>(), st, m, o, n, iters);
-  }
+template <typename Kern, typename... Args>
+int launch_fwd(Kern k, int64_t blocks, int threads, size_t lds, hipStream_t st, Args... args) {
+  if (int s = check_fit(reinterpret_cast<const void*>(k), threads, lds, "newton forward")) return s;
+  if (int s = set_lds(k, lds)) return s;
+  hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(threads), lds, st, args...);
   return check_launch("newton forward");
+}
+
+// NP = 16 ceil(n / 16). n <= 16: one fp32 wave. 16 < n <= 64: the four-wave (NP / 16)
+// kernel of 16-column strips, whose waves hold a quarter of the work each; from two
+// matrices per CU on, NP = 64 takes the two-wave one of 32-column strips, whose 32 x 32
+// products leave the SIMD to the splitting (1024 x 64^2, 12 iterations: 70.0 against
+// 59.5 us, 512: 42 against 29.5; below, a matrix's latency counts: 32 matrices 18.9 us).
+// n > 64: one workgroup of 32-column waves per matrix and CU.
+template <typename T, int NP>
+int fwd_np(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
+  const bool many = bh >= 2 * (int64_t)num_cus();
+  // fp32 n = 49: the symmetric iteration when P is symmetric (the kernel checks; else the general one).
+  if constexpr (std::is_same<T, float>::value && NP == 64)
+    if (n == 49)
+      return many ? launch_fwd(newton_fwd_sym_kernel<8>, bh, 512, fwd_lds<NP>(), st, m, o, n, iters)
+                  : launch_fwd(newton_fwd_sym_kernel<16>, bh, 1024, fwd_lds<NP>(), st, m, o, n, iters);
+  if constexpr (NP == 16) {
+    return launch_fwd(newton_fwd_kernel<T, NP>, bh, NP * 4, fwd_lds<NP>(), st, m, o, n, iters);
+  } else if constexpr (NP <= 64) {
+    constexpr int NT = NP / 16;
+    if constexpr (NP == 64)
+      if (many)
+        return launch_fwd(newton_fwd_tile_kernel<T>, (bh + 1) / 2, 256, 2 * TileLayout::LDS, st, m, o, bh, n, iters);
+    return launch_fwd(newton_fwd_chain_kernel<T, NT>, bh, 64 * NT, ChainLayout<NT>::LDS, st, m, o, n, iters);
+  } else {
+    constexpr int NR = (NP + 31) / 32, KS = std::is_same<T, float>::value ? NP / 16 : 2 * NR;
+    return launch_fwd(newton_fwd_wide_kernel<T, NR, KS>, bh, 64 * NR, WideLayout<NR, KS>::LDS, st, m, o, n, iters);
+  }
 }
 
 // 64 x 64 fp32 matrices, 2 to 8 per CU: the persistent issue-ordered kernel (1024 x 64^2:
@@ -1646,16 +1635,7 @@ int bwd_np_w(const T* g, const T* v, T* o, int64_t bh, int n, hipStream_t st) {
   return check_launch("newton backward");
 }
 
-// Four waves per strip only while there are fewer than two matrices per CU
-// (latency-bound); with more, two per strip keep more matrices resident.
-template <int NP> bool use_wide(int64_t bh) { return pick_wpr<NP>() == 4 && bh < 2 * (int64_t)num_cus(); }
 template <int NP> constexpr int narrow_wpr() { return pick_wpr<NP>() == 4 ? 2 : pick_wpr<NP>(); }
-
-template <typename T, int NP>
-int fwd_np(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
-  if (use_wide<NP>(bh)) return fwd_np_w<T, NP, pick_wpr<NP>()>(m, o, bh, n, iters, st);
-  return fwd_np_w<T, NP, narrow_wpr<NP>()>(m, o, bh, n, iters, st);
-}
 
 // The backward's two products per matrix are latency-bound at any matrix count
 // (four waves per strip: 14.5 against 15.2 us at 1024 x 64^2, where the forward's

@@ -299,3 +299,40 @@ def test_newton_config4(gpu):
     ref = oracle.newton_forward(A, 16, "f32")
     assert_newton_close(V, ref, "f32", "cfg4 fwd")
     assert_newton_close(dA, oracle.newton_backward(G, V.cpu(), "f32"), "f32", "cfg4 bwd", rtol=1e-5)
+
+
+@pytest.mark.parametrize("bh,n,dt", [(511, 64, "f32"), (512, 64, "f32"), (513, 50, "f32"), (515, 63, "f16"),
+                                     (3, 33, "f32"), (2, 47, "bf16"), (2, 81, "f32"), (2, 97, "bf16"), (2, 127, "f16")])
+@pytest.mark.parametrize("iters", [0, 1, 2, 9])
+def test_newton_forward_split(gpu, bh, n, dt, iters):
+    """The bf16-piece iterations at the edges of their size and count rules: two matrices to a
+    workgroup (512 and more of 48 < n <= 64, an odd last one), one 16-column strip per wave
+    (fewer), one workgroup per matrix above 64; general matrices, whose iterates are not
+    symmetric, so that a transposed tile would show."""
+    import laplacianformer_amd as lf
+
+    print(f"newton forward split bh={bh} n={n} {dt} iters={iters}", flush=True)
+    A = gram(1, n, 64, seed=900 + n)
+    noise = gen((bh, n, n), 901 + n, "f64").numpy()
+    A = torch.from_numpy(A + 1e-2 / n * noise).reshape(bh, 1, n, n).to(TORCH_DT[dt])
+    out = torch.full_like(A, float("nan"), device=gpu)
+    lf.ext().NewtonInverse_forward(A.to(gpu), out, iters)
+    assert_newton_close(out, oracle.newton_forward(A, iters, dt), dt, f"bh={bh} n={n} {dt} it={iters}")
+
+
+@pytest.mark.parametrize("bh,n", [(2, 40), (2, 64), (600, 64), (2, 100), (2, 128)])
+def test_newton_forward_split_nonfinite(gpu, bh, n):
+    """A matrix with a NaN or an infinity gives no finite value after an iteration (every row
+    and column of the products meets it); the other matrices of the batch are untouched."""
+    import laplacianformer_amd as lf
+
+    print(f"newton forward non-finite bh={bh} n={n}", flush=True)
+    A = torch.from_numpy(gram(bh, n, 64, seed=950 + n)).float().reshape(bh, 1, n, n)
+    bad = A.clone()
+    bad[0, 0, 3, 5] = float("nan")
+    bad[1, 0, n - 1, 2] = float("inf")
+    good, got = torch.empty_like(A, device=gpu), torch.empty_like(A, device=gpu)
+    lf.ext().NewtonInverse_forward(A.to(gpu), good, 3)
+    lf.ext().NewtonInverse_forward(bad.to(gpu), got, 3)
+    assert not torch.isfinite(got[:2]).any()
+    assert torch.equal(got[2:], good[2:])
