@@ -1198,7 +1198,6 @@ newton_bwd_f64_kernel(const double* __restrict__ gout, const double* __restrict_
 // NP = 64*ceil(n/64):  T = P V,  V' = 2V - V T  (the V(PV) order, ping-pong V).
 // ---------------------------------------------------------------------------
 constexpr int kBgTile = 64;  // padding granule of NP (and the smallest workgroup tile side)
-constexpr int kBgK = 16;     // k per LDS stage
 
 constexpr int kBgMaxNP = 256;  // largest padded size of the GEMM path
 constexpr int kInitRows = 16;  // rows per workgroup of the init kernel
@@ -1230,6 +1229,7 @@ newton_big_init_kernel(const T* __restrict__ mat, float* __restrict__ P, float* 
     float sum = -3.4e38f;
     if (i < n) {
       sum = 0.0f;
+#pragma unroll 16
       for (int j = 0; j < n; ++j) sum += rows[threadIdx.x][j];
     }
     rowsum[m * NP + i] = sum;
@@ -1275,155 +1275,6 @@ newton_big_unpack_kernel(const float* __restrict__ src, T* __restrict__ dst, con
   dst[m * n * n + e] = from_acc<T>(scale * src[m * NP * NP + (size_t)i * NP + j]);
 }
 
-// Batched D = f(op(X) op(Y)) over NP x NP fp32 matrices (row-major, matrix
-// stride NP*NP), op = transpose when TX / TY. MODE 0: D = XY; 1: D = 2E - XY;
-// 2: D = -XY. SCALED multiplies the result by the matrix's alpha (from the
-// init kernel's row sums). One TM x TN output tile per 4-wave workgroup (2 x 2
-// waves of TM/2 x TN/2). Grid: (NP/TM)(NP/TN) tiles x matrices, flattened so that
-// all tiles of a matrix share blockIdx.x mod 8 (workgroups are dealt to the 8
-// XCDs round robin, so a matrix's tiles share one L2). Both operands are staged
-// k-major in LDS ([k][TM], [k][TN]) with the columns of row k XOR-swizzled by
-// 16 * ((k + k/4) mod 4): the 4 k rows of an MFMA operand read then fall on 4
-// different 16-bank groups, and so do the 4 rows of a transposing store
-// (conflict-free both ways, no padding). Two LDS stages, one
-// barrier per stage; global loads run two stages ahead of the MFMAs through
-// two register sets, so each load has two stages of MFMA work to land in.
-template <int TM, int TN, bool TX, bool TY, int MODE, bool SCALED>
-__global__ void __launch_bounds__(256)
-newton_big_gemm_kernel(const float* __restrict__ X, const float* __restrict__ Y, const float* __restrict__ E,
-                       const float* __restrict__ rowsum, float* __restrict__ D, int NP, int K, int nMat) {
-  static_assert(TM % 64 == 0 && TN % 64 == 0, "tile sides are multiples of 64");
-  constexpr int RT = TM / 32, CT = TN / 32;     // 16x16 accumulators per wave (2 x 2 waves)
-  constexpr int LA = TM / 64, LB = TN / 64;     // float4 staging loads per thread per operand
-  __shared__ __align__(16) float As[2][kBgK][TM];
-  __shared__ __align__(16) float Bs[2][kBgK][TN];
-  auto sw = [](int k) { return 16 * ((k + (k >> 2)) & 3); };
-  const int ntm = NP / TM, ntn = NP / TN;
-  const int tiles = ntm * ntn;
-  // Inverse of the flattening: id = (m % 8) + 8 * (t + tiles * (m / 8)).
-  const int id = blockIdx.x;
-  const int lo = id & 7, hi = id >> 3;
-  const int t = hi % tiles, mg = hi / tiles;
-  const int m = mg * 8 + lo;
-  if (m >= nMat) return;  // whole workgroup
-  const int ti = t / ntn, tj = t - ti * ntn;
-  const size_t mo = (size_t)m * NP * NP;
-  const float* Xm = X + mo;
-  const float* Ym = Y + mo;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wr = (wave >> 1) * (TM / 2), wc = (wave & 1) * (TN / 2);
-  float alpha = 1.0f;
-  if constexpr (SCALED) alpha = big_alpha(rowsum + (size_t)m * NP, NP);
-
-  // Global -> register staging of one k stage: TM x 16 of op(X) and 16 x TN of op(Y).
-  auto load = [&](float4 (&ra)[LA], float4 (&rb)[LB], int k0) {
-#pragma unroll
-    for (int u = 0; u < LA; ++u) {
-      if (TX) {  // A[i][k] = X[k][i]: 16 rows of X, TM contiguous columns
-        const int e = tid + 256 * u, k = e / (TM / 4), iq = (e % (TM / 4)) * 4;
-        ra[u] = *reinterpret_cast<const float4*>(Xm + (size_t)(k0 + k) * NP + ti * TM + iq);
-      } else {   // A[i][k] = X[i][k]: TM rows of X, 16 contiguous columns
-        const int i = (tid >> 2) + 64 * u, kq = (tid & 3) * 4;
-        ra[u] = *reinterpret_cast<const float4*>(Xm + (size_t)(ti * TM + i) * NP + k0 + kq);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < LB; ++u) {
-      if (TY) {  // B[k][j] = Y[j][k]
-        const int j = (tid >> 2) + 64 * u, kq = (tid & 3) * 4;
-        rb[u] = *reinterpret_cast<const float4*>(Ym + (size_t)(tj * TN + j) * NP + k0 + kq);
-      } else {   // B[k][j] = Y[k][j]
-        const int e = tid + 256 * u, k = e / (TN / 4), jq = (e % (TN / 4)) * 4;
-        rb[u] = *reinterpret_cast<const float4*>(Ym + (size_t)(k0 + k) * NP + tj * TN + jq);
-      }
-    }
-  };
-  auto store = [&](const float4 (&ra)[LA], const float4 (&rb)[LB], int b) {
-#pragma unroll
-    for (int u = 0; u < LA; ++u) {
-      if (TX) {
-        const int e = tid + 256 * u, k = e / (TM / 4), iq = (e % (TM / 4)) * 4;
-        *reinterpret_cast<float4*>(&As[b][k][iq ^ sw(k)]) = ra[u];
-      } else {
-        const int i = (tid >> 2) + 64 * u, kq = (tid & 3) * 4;
-        As[b][kq + 0][i ^ sw(kq + 0)] = ra[u].x; As[b][kq + 1][i ^ sw(kq + 1)] = ra[u].y;
-        As[b][kq + 2][i ^ sw(kq + 2)] = ra[u].z; As[b][kq + 3][i ^ sw(kq + 3)] = ra[u].w;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < LB; ++u) {
-      if (TY) {
-        const int j = (tid >> 2) + 64 * u, kq = (tid & 3) * 4;
-        Bs[b][kq + 0][j ^ sw(kq + 0)] = rb[u].x; Bs[b][kq + 1][j ^ sw(kq + 1)] = rb[u].y;
-        Bs[b][kq + 2][j ^ sw(kq + 2)] = rb[u].z; Bs[b][kq + 3][j ^ sw(kq + 3)] = rb[u].w;
-      } else {
-        const int e = tid + 256 * u, k = e / (TN / 4), jq = (e % (TN / 4)) * 4;
-        *reinterpret_cast<float4*>(&Bs[b][k][jq ^ sw(k)]) = rb[u];
-      }
-    }
-  };
-
-  v4f acc[RT][CT];
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) acc[r][c] = v4f{0.f, 0.f, 0.f, 0.f};
-  const int li = lane & 15, lk = lane >> 4;
-  auto compute = [&](int b) {
-#pragma unroll
-    for (int ks = 0; ks < kBgK; ks += 4) {
-      float a[RT], bb[CT];
-#pragma unroll
-      for (int r = 0; r < RT; ++r) a[r] = As[b][ks + lk][(wr + 16 * r + li) ^ sw(ks + lk)];
-#pragma unroll
-      for (int c = 0; c < CT; ++c) bb[c] = Bs[b][ks + lk][(wc + 16 * c + li) ^ sw(ks + lk)];
-#pragma unroll
-      for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], bb[c], acc[r][c], 0, 0, 0);
-    }
-  };
-
-  // The products run over k < K = 32 * ceil(n / 32) <= NP (columns and rows from n
-  // on are zero padding and contribute nothing). nk = K / 16 is even: stages go in
-  // pairs, even stages through LDS buffer 0 and register set 0, odd ones through
-  // buffer 1 and set 1.
-  const int nk = K / kBgK;
-  float4 ra0[LA], rb0[LB], ra1[LA], rb1[LB];
-  load(ra0, rb0, 0);
-  load(ra1, rb1, kBgK);
-  store(ra0, rb0, 0);
-  __syncthreads();
-  for (int kc = 0; kc < nk; kc += 2) {
-    if (kc + 2 < nk) load(ra0, rb0, (kc + 2) * kBgK);
-    compute(0);
-    store(ra1, rb1, 1);
-    __syncthreads();
-    if (kc + 3 < nk) load(ra1, rb1, (kc + 3) * kBgK);
-    compute(1);
-    if (kc + 2 < nk) store(ra0, rb0, 0);
-    __syncthreads();
-  }
-
-  float* Dm = D + mo;
-  const float* Em = MODE == 1 ? E + mo : nullptr;
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int c = 0; c < CT; ++c)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int i = ti * TM + wr + 16 * r + 4 * lk + q;
-        const int j = tj * TN + wc + 16 * c + li;
-        const size_t o = (size_t)i * NP + j;
-        float v = acc[r][c][q];
-        if (MODE == 1) v = 2.0f * Em[o] - v;
-        if (MODE == 2) v = -v;
-        if (SCALED) v = alpha * v;
-        Dm[o] = v;
-      }
-}
-
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
@@ -1459,19 +1310,25 @@ bool big_direct(int n, int np, std::initializer_list<const void*> ptrs) {
   return true;
 }
 
-// Tiles: 128 x 64 for the forward's products (neither operand transposed) when
-// 128 divides NP, measured 10 % faster than 64 x 64 at 128 x 256^2; 64 x 64
-// otherwise (the backward's transposed products measured 15 % slower at 128 x 64).
+template <int TM, int TN, bool TX, bool TY, int MODE, bool SCALED>
+int big_gemm_t(const float* X, const float* Y, const float* E, const float* rowsum, float* D, int np, int K, int64_t bh,
+               hipStream_t st) {
+  auto k = newton_gemm_kernel<TM, TN, TX, TY, MODE, SCALED>;
+  constexpr int lds = gm_lds<TM, TN>();
+  if (int s = check_fit(reinterpret_cast<const void*>(k), 256, lds, "newton products")) return s;
+  if (int s = set_dyn_lds(reinterpret_cast<const void*>(k), lds, "newton products")) return s;
+  hipLaunchKernelGGL(k, dim3(big_gemm_blocks(np, TM, TN, bh)), dim3(256), lds, st, X, Y, E, rowsum, D, np, K, (int)bh);
+  return check_launch("newton products");
+}
+
+// Tiles: 128 x 128 where they divide NP and give every CU one; else 64 x 64.
 template <int MODE, bool SCALED, bool TX = false, bool TY = false>
-void big_gemm(const float* X, const float* Y, const float* E, const float* rowsum, float* D, int np, int n,
-              int64_t bh, hipStream_t st) {
+int big_gemm(const float* X, const float* Y, const float* E, const float* rowsum, float* D, int np, int n, int64_t bh,
+             hipStream_t st) {
   const int K = std::min(np, (n + 31) / 32 * 32);
-  if (!TX && !TY && np % 128 == 0)
-    hipLaunchKernelGGL((newton_big_gemm_kernel<128, 64, TX, TY, MODE, SCALED>),
-                       dim3(big_gemm_blocks(np, 128, 64, bh)), dim3(256), 0, st, X, Y, E, rowsum, D, np, K, (int)bh);
-  else
-    hipLaunchKernelGGL((newton_big_gemm_kernel<64, 64, TX, TY, MODE, SCALED>),
-                       dim3(big_gemm_blocks(np, 64, 64, bh)), dim3(256), 0, st, X, Y, E, rowsum, D, np, K, (int)bh);
+  if (np % 128 == 0 && bh * (np / 128) * (np / 128) >= num_cus())
+    return big_gemm_t<128, 128, TX, TY, MODE, SCALED>(X, Y, E, rowsum, D, np, K, bh, st);
+  return big_gemm_t<64, 64, TX, TY, MODE, SCALED>(X, Y, E, rowsum, D, np, K, bh, st);
 }
 
 template <typename T>
@@ -1496,13 +1353,13 @@ int big_fwd(const T* mat, T* out, int64_t bh, int n, int iters, float* ws, hipSt
   for (int it = 0; it < iters; ++it) {
     float* dst = (direct && it == iters - 1) ? reinterpret_cast<float*>(out) : Vb;
     if (it == 0) {  // V0 = alpha P:  T = alpha (P P),  V1 = alpha (2P - P T)
-      big_gemm<0, true>(P, P, nullptr, rs, Tm, np, n, bh, st);
-      big_gemm<1, true>(P, Tm, P, rs, dst, np, n, bh, st);
+      s = big_gemm<0, true>(P, P, nullptr, rs, Tm, np, n, bh, st);
+      if (!s) s = big_gemm<1, true>(P, Tm, P, rs, dst, np, n, bh, st);
     } else {        // T = P V,  V' = 2V - V T
-      big_gemm<0, false>(P, Va, nullptr, nullptr, Tm, np, n, bh, st);
-      big_gemm<1, false>(Va, Tm, Va, nullptr, dst, np, n, bh, st);
+      s = big_gemm<0, false>(P, Va, nullptr, nullptr, Tm, np, n, bh, st);
+      if (!s) s = big_gemm<1, false>(Va, Tm, Va, nullptr, dst, np, n, bh, st);
     }
-    if ((s = check_launch("newton forward step"))) return s;
+    if (s) return s;
     std::swap(Va, Vb);
   }
   if (direct) return LFAMD_OK;
@@ -1522,18 +1379,17 @@ int big_bwd(const T* g, const T* inv, T* out, int64_t bh, int n, float* ws, hipS
   const bool apart = o + bytes <= v || v + bytes <= o;
   if (apart && big_direct<T>(n, np, {g, inv, out})) {  // S = V^T G,  out = -S V^T
     const float* Vf = reinterpret_cast<const float*>(inv);
-    big_gemm<0, false, true, false>(Vf, reinterpret_cast<const float*>(g), nullptr, nullptr, S, np, n, bh, st);
-    big_gemm<2, false, false, true>(S, Vf, nullptr, nullptr, reinterpret_cast<float*>(out), np, n, bh, st);
-    return check_launch("newton backward products");
+    if (int s = big_gemm<0, false, true, false>(Vf, reinterpret_cast<const float*>(g), nullptr, nullptr, S, np, n, bh, st))
+      return s;
+    return big_gemm<2, false, false, true>(S, Vf, nullptr, nullptr, reinterpret_cast<float*>(out), np, n, bh, st);
   }
   float* Vf = ws;
   float* Gf = ws + (size_t)bh * mat_elems;
   dim3 pg(ceil_div(np * np, 256), (unsigned)bh);
   hipLaunchKernelGGL(newton_big_pack_kernel<T>, pg, dim3(256), 0, st, inv, Vf, n, np);
   hipLaunchKernelGGL(newton_big_pack_kernel<T>, pg, dim3(256), 0, st, g, Gf, n, np);
-  big_gemm<0, false, true, false>(Vf, Gf, nullptr, nullptr, S, np, n, bh, st);  // S = V^T G
-  big_gemm<2, false, false, true>(S, Vf, nullptr, nullptr, Gf, np, n, bh, st);  // -S V^T (into G's slot)
-  int s = check_launch("newton backward products");
+  int s = big_gemm<0, false, true, false>(Vf, Gf, nullptr, nullptr, S, np, n, bh, st);  // S = V^T G
+  if (!s) s = big_gemm<2, false, false, true>(S, Vf, nullptr, nullptr, Gf, np, n, bh, st);  // -S V^T (into G's slot)
   if (s) return s;
   dim3 ug(ceil_div(n * n, 256), (unsigned)bh);
   hipLaunchKernelGGL((newton_big_unpack_kernel<T, 1, false>), ug, dim3(256), 0, st, Gf, out,

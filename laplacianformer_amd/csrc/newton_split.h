@@ -865,4 +865,234 @@ newton_fwd_wide_kernel(const T* __restrict__ mat, T* __restrict__ out, int n, in
     }
 }
 
+
+// ---------------------------------------------------------------------------
+// Batched D = f(op(X) op(Y)) over NP x NP fp32 matrices (row-major, matrix stride
+// NP * NP), op = transpose when TX / TY, on bf16 pieces. MODE 0: D = XY; 1: D = 2E - XY;
+// 2: D = -XY. SCALED multiplies the result by the matrix's alpha (from the init
+// kernel's row sums). One TM x TN output tile per workgroup of 2 x 2 waves. Grid: tiles x matrices, flattened so that
+// all tiles of a matrix share blockIdx.x mod 8 (workgroups are dealt to the 8 XCDs
+// round robin, so a matrix's tiles share one L2).
+//
+// Both operands are staged 32 k at a time, split on the way into their pieces in MFMA
+// operand order (two buffers, one barrier per 32 k, global loads two stages ahead):
+// each element is split once per tile that reads it, 4 VALU instructions to an MFMA,
+// and the stages of that go between the matrix instructions.
+//
+// Staging by rows (op(X)[i][k] with k contiguous): a lane has four k of one row.
+// By columns (k strided): a lane has four k of JB = T / 32 neighbouring rows or
+// columns of the operand. Either way four k of one row are 8 bytes of an operand slot;
+// the slot of row l is permuted so that a half wave's 32 writes fall on 64 banks.
+// ---------------------------------------------------------------------------
+constexpr int kGmK = 32;  // k per stage
+
+// Slot (of 64 16-byte ones) of row l, half h of step s in row tile `tile`.
+template <int T, bool COLS> __device__ __forceinline__ int gm_slot(int l, int h, int s, int tile) {
+  if constexpr (!COLS) return (l ^ (4 * h + 8 * s)) + 32 * h;
+  else if constexpr (T == 128) return (((l & 3) * 8 + (l >> 2)) ^ (8 * (tile & 1))) + 32 * h;
+  else return ((l & 1) * 16 + (l >> 1)) + 32 * h;
+}
+
+// One operand's staging of a workgroup: T rows (or columns) x 32 k per stage.
+template <int T, bool COLS> struct GmStage {
+  static constexpr int Q = T / 32;  // quads (four k of one row) per thread
+  using Regs = float4[COLS ? 4 : Q];  // COLS: row k of the quad, Q columns (x, y for T = 64)
+  int goff, loff[Q];
+  __device__ __forceinline__ GmStage(int tid, int NP) {
+    const int w = tid >> 6, lane = tid & 63;
+    if constexpr (!COLS) {
+      const int f = tid & 7, row = tid >> 3;  // 32 rows a pass
+      goff = row * NP + 4 * f;
+      const int s = f >> 2, c3 = (f >> 1) & 1, h = f & 1;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) loff[q] = (q * 2 + s) * 3072 + gm_slot<T, COLS>(row, h, s, q) * 16 + 8 * c3;
+    } else {
+      const int jq = (lane & 15) + 16 * (w & 1), c3 = (lane >> 4) & 1, h = lane >> 5, s = w >> 1;
+      goff = (16 * s + 8 * c3 + 4 * h) * NP + Q * jq;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int j = Q * jq + q;
+        loff[q] = ((j >> 5) * 2 + s) * 3072 + gm_slot<T, COLS>(j & 31, h, s, j >> 5) * 16 + 8 * c3;
+      }
+    }
+  }
+  // Stage k0 of the operand whose rows (COLS: columns) start at `base`.
+  __device__ __forceinline__ void load(Regs& r, const float* __restrict__ base, int NP, int k0) const {
+    if constexpr (!COLS) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) r[q] = *reinterpret_cast<const float4*>(base + (unsigned)(goff + 32 * q * NP + k0));
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float* p = base + (unsigned)(goff + (k0 + k) * NP);
+        if constexpr (Q == 4) {
+          r[k] = *reinterpret_cast<const float4*>(p);
+        } else {
+          const float2 v = *reinterpret_cast<const float2*>(p);
+          r[k].x = v.x;
+          r[k].y = v.y;
+        }
+      }
+    }
+  }
+  static __device__ __forceinline__ float at(const Regs& r, int q, int k) {
+    if constexpr (!COLS) return k == 0 ? r[q].x : k == 1 ? r[q].y : k == 2 ? r[q].z : r[q].w;
+    else return q == 0 ? r[k].x : q == 1 ? r[k].y : q == 2 ? r[k].z : r[k].w;
+  }
+};
+
+template <int TM, int TN> constexpr int gm_lds() { return 2 * (TM + TN) * kGmK * 3 * 2; }
+
+template <int TM, int TN, bool TX, bool TY, int MODE, bool SCALED>
+__global__ void __launch_bounds__(256)
+newton_gemm_kernel(const float* __restrict__ X, const float* __restrict__ Y, const float* __restrict__ E,
+                   const float* __restrict__ rowsum, float* __restrict__ D, int NP, int K, int nMat) {
+  constexpr int RT = TM / 64, CT = TN / 64;  // 32 x 32 tiles per wave
+  extern __shared__ __align__(16) unsigned char gm_sm[];
+  constexpr int ABYTES = TM * kGmK * 6, BUF = (TM + TN) * kGmK * 6;
+  const int ntm = NP / TM, ntn = NP / TN, tiles = ntm * ntn;
+  const int id = blockIdx.x, hi = id >> 3;  // id = (m % 8) + 8 (t + tiles (m / 8))
+  const int t = hi % tiles, m = hi / tiles * 8 + (id & 7);
+  if (m >= nMat) return;  // whole workgroup
+  const int ti = t / ntn, tj = t - ti * ntn;
+  const size_t mo = (size_t)m * NP * NP;
+  const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = tid & 63, li = lane & 31, lh = lane >> 5;
+  const int wr = wave >> 1, wc = wave & 1;
+  GmStage<TM, TX> sa(tid, NP);
+  GmStage<TN, !TY> sb(tid, NP);
+  const float* Xb = X + mo + (TX ? (size_t)ti * TM : (size_t)ti * TM * NP);
+  const float* Yb = Y + mo + (TY ? (size_t)tj * TN * NP : (size_t)tj * TN);
+  struct Set {
+    typename GmStage<TM, TX>::Regs a;
+    typename GmStage<TN, !TY>::Regs b;
+  } rg;
+  auto gload = [&](Set& r, int kc) {
+    sa.load(r.a, Xb, NP, kc * kGmK);
+    sb.load(r.b, Yb, NP, kc * kGmK);
+  };
+  // Quad q (A's, then B's) of the staged registers, in four stages, the last one stored to buffer b.
+  constexpr int QA = GmStage<TM, TX>::Q, QB = GmStage<TN, !TY>::Q, QS = QA + QB;
+  uint32_t d0[3], d1[3];
+  float y[4];
+  auto stage = [&](const Set& rs, int i, int b) {
+    const int q = i / 4;
+    auto put = [&](int pc) {
+      d0[pc] = bf16_pair(y[0], y[1]);
+      d1[pc] = bf16_pair(y[2], y[3]);
+    };
+    auto drop = [&](int pc) {
+      y[0] -= __builtin_bit_cast(float, d0[pc] << 16);
+      y[1] -= __builtin_bit_cast(float, d0[pc] & 0xffff0000u);
+      y[2] -= __builtin_bit_cast(float, d1[pc] << 16);
+      y[3] -= __builtin_bit_cast(float, d1[pc] & 0xffff0000u);
+    };
+    if (i % 4 == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) y[k] = q < QA ? sa.at(rs.a, q < QA ? q : 0, k) : sb.at(rs.b, q < QA ? 0 : q - QA, k);
+      put(0);
+    } else if (i % 4 == 1) {
+      drop(0);
+    } else if (i % 4 == 2) {
+      put(1);
+      drop(1);
+    } else {
+      put(2);
+      unsigned char* p = gm_sm + b * BUF + (q < QA ? sa.loff[q < QA ? q : 0] : ABYTES + sb.loff[q < QA ? 0 : q - QA]);
+#pragma unroll
+      for (int pc = 0; pc < 3; ++pc) *reinterpret_cast<uint2*>(p + 1024 * pc) = uint2{d0[pc], d1[pc]};
+    }
+  };
+  const int nk = K / kGmK;
+  gload(rg, 0);
+#pragma unroll
+  for (int i = 0; i < 4 * QS; ++i) stage(rg, i, 0);
+  gload(rg, nk > 1 ? 1 : 0);
+  float alpha = 1.0f;
+  if constexpr (SCALED) {
+    __shared__ float red[4];
+    float v = -3.4e38f;
+    for (int i = tid; i < NP; i += 256) v = fmaxf(v, rowsum[(size_t)m * NP + i]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
+    if (lane == 0) red[wave] = v;
+    __syncthreads();
+    const float mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    alpha = 1.8f / (mx * mx);
+  } else {
+    __syncthreads();
+  }
+  int aoff[2][RT], boff[2][CT];  // this lane's slots, per step
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) aoff[s][r] = ((wr * RT + r) * 2 + s) * 3072 + gm_slot<TM, TX>(li, lh, s, wr * RT + r) * 16;
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+      boff[s][c] = ABYTES + ((wc * CT + c) * 2 + s) * 3072 + gm_slot<TN, !TY>(li, lh, s, wc * CT + c) * 16;
+  }
+  v16f acc[RT][CT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[r][c][q] = 0.f;
+  constexpr int MC = 12 * RT * CT;  // products per stage
+  // Stage kc: the products from buffer kc % 2, between them the next stage's splitting,
+  // at the end the loads of the one after.
+#pragma unroll 1
+  for (int kc = 0; kc < nk; ++kc) {
+    const unsigned char* buf = gm_sm + (kc & 1) * BUF;
+    uint4 xa[2][RT][3], xb[2][CT][3];
+    auto fetch = [&](int s) {
+#pragma unroll
+      for (int pc = 0; pc < 3; ++pc) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) xa[s][r][pc] = *reinterpret_cast<const uint4*>(buf + aoff[s][r] + 1024 * pc);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) xb[s][c][pc] = *reinterpret_cast<const uint4*>(buf + boff[s][c] + 1024 * pc);
+      }
+    };
+    fetch(0);
+    fetch(1);  // (spread over the first step's products instead, 1076 against 982 us at 128 x 256^2)
+    __builtin_amdgcn_sched_barrier(0);
+    unrolled<MC>([&](auto mc) {
+      constexpr int mm = decltype(mc)::value, s = mm / (MC / 2), e = mm % (MC / 2), r = e / 6 / CT, c = e / 6 % CT;
+      acc[r][c] = mfma_piece(xa[s][r], xb[s][c], e % 6, false, acc[r][c]);
+      // (After the last stage's products nobody reads the other buffer.)
+      constexpr int PER = (4 * QS + MC - 5) / (MC - 4);  // stages per product, done before the last products
+      if constexpr (mm >= 2) {
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+          if ((mm - 2) * PER + k < 4 * QS) stage(rg, (mm - 2) * PER + k, (kc + 1) & 1);
+      }
+      if constexpr (mm == MC - 1)
+        if (kc + 2 < nk) gload(rg, kc + 2);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    __syncthreads();
+  }
+
+  float* Dm = D + mo;
+  const float* Em = MODE == 1 ? E + mo : nullptr;
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int i0 = ti * TM + 32 * (wr * RT + r) + 4 * lh, j = tj * TN + 32 * (wc * CT + c) + li;
+      float ev[16];
+      if constexpr (MODE == 1)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) ev[q] = Em[(unsigned)((i0 + 8 * (q >> 2) + (q & 3)) * NP + j)];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        float v = acc[r][c][q];
+        if (MODE == 1) v = 2.0f * ev[q] - v;
+        if (MODE == 2) v = -v;
+        if (SCALED) v = alpha * v;
+        Dm[(unsigned)((i0 + 8 * (q >> 2) + (q & 3)) * NP + j)] = v;
+      }
+    }
+}
+
 }  // namespace lfamd

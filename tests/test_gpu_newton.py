@@ -336,3 +336,20 @@ def test_newton_forward_split_nonfinite(gpu, bh, n):
     lf.ext().NewtonInverse_forward(bad.to(gpu), got, 3)
     assert not torch.isfinite(got[:2]).any()
     assert torch.equal(got[2:], good[2:])
+
+
+@pytest.mark.parametrize("bh,n", [(64, 256), (65, 196), (3, 193), (9, 150)])
+def test_newton_large_split(gpu, bh, n):
+    """The piece products of n > 128 on both tile sizes (128 x 128 where they give every CU one),
+    on general matrices (no symmetric iterate) and gradients; matrix counts off a multiple of 8."""
+    import laplacianformer_amd as lf
+
+    print(f"newton large split bh={bh} n={n}", flush=True)
+    A = gram(1, n, 64, seed=970 + n) + 1e-2 / n * gen((bh, n, n), 971 + n, "f64").numpy()
+    A = torch.from_numpy(A).float().reshape(bh, 1, n, n)
+    out = torch.empty_like(A, device=gpu)
+    lf.ext().NewtonInverse_forward(A.to(gpu), out, 3)
+    assert_newton_close(out, oracle.newton_forward(A, 3, "f32"), "f32", f"bh={bh} n={n}")
+    V, G = gen((bh, 1, n, n), 972 + n, "f32", scale=0.3), gen((bh, 1, n, n), 973 + n, "f32")
+    lf.ext().NewtonInverse_backward(G.to(gpu), V.to(gpu), out)
+    assert_newton_close(out, oracle.newton_backward(G, V, "f32"), "f32", f"bwd bh={bh} n={n}", rtol=1e-5)
