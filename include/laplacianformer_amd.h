@@ -181,6 +181,25 @@ int lfamd_laplace_kernel_backward_multi(int dtype, int num_sources, const float*
                                         int64_t channels, float scale, void* workspace, size_t workspace_bytes,
                                         void* stream);
 
+/* The same for any fp16 / bf16 / fp32 rows and 17 <= M <= 256 or M = 16 (any C):
+ * up to three row sets that share one key, fp32 grad_kernels[i] and kernels[i]
+ * [B,H,q_lens[i],M], queries[i] and grad_queries[i] [B,H,q_lens[i],C], grad_key
+ * [B,H,C,M] summed over the sets with one rounding. 1 <= q_lens[i] <= INT32_MAX / 8,
+ * batch * heads <= 65535; the workspace is
+ * lfamd_laplace_kernel_backward_rows_workspace_size bytes (0 and
+ * LFAMD_ERR_UNSUPPORTED where the path does not apply; callers then compose the
+ * distance's backward). No reference counterpart: the attention layer's call where
+ * the fp16-only entry above does not apply. */
+size_t lfamd_laplace_kernel_backward_rows_workspace_size(int dtype, int num_sources, const int64_t* q_lens,
+                                                         int64_t batch, int64_t heads, int64_t k_len,
+                                                         int64_t channels);
+int lfamd_laplace_kernel_backward_rows(int dtype, int num_sources, const float* const* grad_kernels,
+                                       const float* const* kernels, const void* const* queries,
+                                       const int64_t* q_lens, const void* key, void* const* grad_queries,
+                                       void* grad_key, int64_t batch, int64_t heads, int64_t k_len,
+                                       int64_t channels, float scale, void* workspace, size_t workspace_bytes,
+                                       void* stream);
+
 /* ---- NewtonInverse ------------------------------------------------------ */
 
 /* Bytes of device workspace lfamd_newton_forward / lfamd_newton_backward need:

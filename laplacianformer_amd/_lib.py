@@ -40,6 +40,9 @@ CAPI_PROTOTYPES = [
     ("lfamd_laplace_kernel_backward_multi_workspace_size", _SZ, [_I, _I, _P, _I64, _I64, _I64, _I64]),
     ("lfamd_laplace_kernel_backward_multi", _I, [_I, _I, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64,
                                                   ctypes.c_float, _P, _SZ, _P]),
+    ("lfamd_laplace_kernel_backward_rows_workspace_size", _SZ, [_I, _I, _P, _I64, _I64, _I64, _I64]),
+    ("lfamd_laplace_kernel_backward_rows", _I, [_I, _I, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64,
+                                                  ctypes.c_float, _P, _SZ, _P]),
     ("lfamd_newton_workspace_size", _SZ, [_I, _I64, _I64]),
     ("lfamd_newton_forward", _I, [_I, _P, _P, _I64, _I64, _I, _P, _SZ, _P]),
     ("lfamd_newton_backward", _I, [_I, _P, _P, _P, _I64, _I64, _P, _SZ, _P]),

@@ -674,37 +674,55 @@ laplace_bwd_kernel(const T* __restrict__ gout, const T* __restrict__ query,
 constexpr int kBcRB = 8;  // grad rows per LDS batch
 constexpr int kBcBufs = 4;  // LDS accumulators of the workgroup grad_key reduction
 
+// fp32 steps y = (sgn(q - k) + 1)/2 of the two backward kernels below. A workgroup whose
+// keys are all below 2^103 scales keys and queries by 2^24: exact, a key cannot overflow,
+// and a query that does is an infinity on its own side of every key. A nonzero scaled
+// difference is then at least 2^-125 and one FMA by 2^126 takes it past the clamp: a
+// subtraction and a clamped FMA. With larger keys (infinities, NaN) the plain difference
+// is scaled twice by 2^100 (>= 2^-149 becomes >= 2^51), one instruction more.
+// Both loops are compiled where a kernel computes one gradient of a plain grad_output
+// (fp32, 32 slices, N = 3136, M = 49, C = 64: grad_query 40 -> 33 us); with both
+// gradients the second loop's registers spill (55 -> 93 us with it), and those keep the
+// unscaled step alone.
+constexpr float kStepKeyMax = 0x1p103f, kStepPre = 0x1p24f, kStepFast = 0x1p126f, kStepSlow = 0x1p100f;
+
+// Floats of the key tile [mc][65], whole 16-byte groups.
+__host__ __device__ constexpr int bcast_key_floats(int mc) { return (mc * 65 + 3) & ~3; }
+
 // Workgroup sum of the per-wave grad_key partials v[MC] (lane = channel), in a
 // fixed order: wave w adds into LDS accumulator w % kBcBufs in rounds of
 // increasing w / kBcBufs, then the accumulators are summed 0, 1, ... and the
-// result is written to `out` column-major, [MC][64] (channel fastest: LDS reads
-// without bank conflicts, coalesced stores). Every read of a round is issued
-// before its writes. Needs kBcBufs * MC * 64 floats of LDS at `red`.
-template <int MC>
+// result goes to out(column, channel, sum), consecutive threads on consecutive
+// channels, or with `cols` on consecutive columns (the pitch of 65 keeps both walks of
+// the LDS and both stores coalesced). Every read of a round is issued before its
+// writes. Needs kBcBufs * bcast_key_floats(MC) floats of LDS at `red`.
+template <int MC, typename Out>
 __device__ __forceinline__ void bcast_reduce_dk(const float (&v)[MC], float* red, int W, int wave, int lane,
-                                                float* __restrict__ out) {
+                                                bool cols, Out out) {
+  constexpr int BF = bcast_key_floats(MC);
   const int nb = min(W, kBcBufs);
-  float* buf = red + (wave % nb) * MC * 64;
+  float* buf = red + (wave % nb) * BF;
   __syncthreads();  // every wave is done with the LDS it used before
   for (int round = 0; round * nb < W; ++round) {
     if (wave / nb == round) {
       if (round == 0) {
 #pragma unroll
-        for (int j = 0; j < MC; ++j) buf[j * 64 + lane] = v[j];
+        for (int j = 0; j < MC; ++j) buf[j * 65 + lane] = v[j];
       } else {
         float pv[MC];
 #pragma unroll
-        for (int j = 0; j < MC; ++j) pv[j] = buf[j * 64 + lane];
+        for (int j = 0; j < MC; ++j) pv[j] = buf[j * 65 + lane];
 #pragma unroll
-        for (int j = 0; j < MC; ++j) buf[j * 64 + lane] = pv[j] + v[j];
+        for (int j = 0; j < MC; ++j) buf[j * 65 + lane] = pv[j] + v[j];
       }
     }
     __syncthreads();
   }
   for (int t = threadIdx.x; t < 64 * MC; t += blockDim.x) {
-    float s = red[t];
-    for (int b = 1; b < nb; ++b) s += red[b * MC * 64 + t];
-    out[t] = s;
+    const int j = cols ? t % MC : t >> 6, cl = cols ? t / MC : t & 63;
+    float s = red[j * 65 + cl];
+    for (int b = 1; b < nb; ++b) s += red[b * BF + j * 65 + cl];
+    out(j, cl, s);
   }
 }
 
@@ -713,22 +731,56 @@ __host__ __device__ constexpr int bcast_max_waves(int mc) { return mc <= 16 ? 16
 // of them (the row loop keeps two groups in flight in a two-slot ring).
 __host__ __device__ constexpr int bcast_pitch(int mc) { return (mc + 7) & ~7; }
 
-// Where the backward's grad_output comes from: fp16 elements, or (LaplacianFormer's
+// Where the backward's grad_output comes from: its elements, or (LaplacianFormer's
 // kernel K = exp(-s * dist)) the gradient of K in fp32 together with K, from which
 // the distance's gradient g = -s * gK * K is formed while a batch is staged.
 enum BwdGrad { kGradF16 = 0, kGradKernel = 1 };
 
-template <typename T, int MC, bool DQ, bool DK, int GSRC = kGradF16>
+// Whether a backward kernel compiles both fp32 step loops (kStepFast).
+template <typename T, bool DQ, bool DK, int GSRC>
+constexpr bool two_step_loops() { return sizeof(T) == 4 && !(DQ && DK) && GSRC == kGradF16; }
+
+// The kernel-gradient backward's rows: up to three row sets (a layer's K_mm, K_qm and
+// K_km share one key) taken as one concatenation, set i ending at row (column-block
+// kernel: row batch) end[i]; unused sets are empty. One launch and one grad_key
+// reduction replace one of each per set, and the waves' shares stay even whatever the
+// sets' lengths.
+struct RowSources {
+  const float* gk[3];
+  const float* kv[3];
+  const void* q[3];
+  void* dq[3];
+  int len[3];
+  int end[3];
+};
+
+// A batch of rows: set s, first row `row` of it, nr rows.
+struct RowBatch {
+  int s, row, nr;
+};
+
+// (A select per use, not an indexed load: the set is uniform and the struct stays in
+// the kernel's arguments.)
+template <typename P>
+__device__ __forceinline__ P pick3(const P (&a)[3], int s) {
+  return s == 0 ? a[0] : s == 1 ? a[1] : a[2];
+}
+
+// RPW = 2 (C <= 32): a wave's halves take two rows at once, lane (h, c) channel c of
+// row 2i + h, where one row would leave half the lanes idle; the halves' grad_key sums
+// are added at the end.
+template <typename T, int MC, bool DQ, bool DK, int GSRC = kGradF16, int RPW = 1>
 __global__ void __launch_bounds__(64 * bcast_max_waves(MC))
-laplace_bwd_bcast_kernel(const T* __restrict__ gout, const float* __restrict__ gkern,
-                         const float* __restrict__ kern, float gscale, const T* __restrict__ query,
+laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscale, const T* __restrict__ query,
                          const T* __restrict__ key, T* __restrict__ dq, T* __restrict__ dk,
                          float* __restrict__ partial, int N, int C, int rowsPerWave) {
   constexpr int RB = kBcRB;
   constexpr int MP = bcast_pitch(MC);            // LDS row pitch (floats)
   constexpr bool kF16 = std::is_same<T, f16s>::value;
+  // 16-bit inputs take the ordered-pattern step (tmap16): y = clamp(T(q) + (1/2 - T(k))).
+  constexpr bool k16 = sizeof(T) == 2;
+  constexpr bool kTwo = two_step_loops<T, DQ, DK, GSRC>();
   constexpr int EPW = sizeof(T) == 2 ? 2 : 1;    // grad elements per 32-bit word
-  static_assert(GSRC == kGradF16 || kF16, "the kernel-gradient source is instantiated for fp16 only");
   constexpr int GD = GSRC == kGradF16 ? RB * MC / EPW : RB * MC;  // grad words of a full batch
   constexpr int NL = (GD + 63) / 64;             // words per lane per batch
   const int W = blockDim.x >> 6;
@@ -736,20 +788,20 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, const float* __restrict__ g
   const int lane = threadIdx.x & 63;
   const int bh = blockIdx.z, cb = blockIdx.y, x = blockIdx.x, nx = gridDim.x;
   const int slice = bh * gridDim.y + cb;
-  const int c = cb * 64 + lane;
+  const int hr = RPW == 2 ? lane >> 5 : 0, ln = RPW == 2 ? lane & 31 : lane;  // row of a pair, channel of the block
+  const int c = cb * 64 + ln;
   const bool cval = c < C;
   const int rowBeg = uniform((x * W + wave) * rowsPerWave);
-  const int rowEnd = uniform(min(N, rowBeg + rowsPerWave));
+  const int rowEnd = uniform(min(GSRC == kGradKernel ? src.end[2] : N, rowBeg + rowsPerWave));
 
   extern __shared__ __align__(16) unsigned char smem[];
-  float* ksm = reinterpret_cast<float*>(smem);             // [MC][64] key tile, then grad_key sums
-  // This wave's batch: [RB][MP] 2g, [RB] -sum_j g, [MP] column sums, [RB][64] scaled query.
-  float* gsm = ksm + MC * 64 + wave * (RB * MP + RB + MP + RB * 64);
+  float* ksm = reinterpret_cast<float*>(smem);             // [MC][65] key tile, then grad_key sums
+  // This wave's batch: [RB][MP] 2g, [RB] -sum_j g, [MP] column sums, [RB / RPW][64] query.
+  float* gsm = ksm + bcast_key_floats(MC) + wave * (RB * MP + RB + MP + RB / RPW * 64);
   float* gneg = gsm + RB * MP;
   float* hsm = gneg + RB;
   float* qsm = hsm + MP;
 
-  const T* qb = query + (size_t)bh * N * C;
   const uint32_t* gw = reinterpret_cast<const uint32_t*>(gout + (size_t)bh * N * MC);
   const T* kb = key + (size_t)bh * C * MC;
 
@@ -757,22 +809,36 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, const float* __restrict__ g
   float kpre[GSRC == kGradKernel ? NL : 1];
   const float gscale2 = -2.0f * gscale;  // 2 * (-s * gK) * K == (-2s * gK) * K exactly
   int kwords = 0;                        // valid words of the fetched kernel-gradient batch
-  T qpre[RB];
-  auto fetch = [&](int rb) {
+  T qpre[RB / RPW];
+  // The batch at row `pos` of the concatenation: it ends with its set. (N is the only
+  // set of a plain grad_output.)
+  auto locate = [&](int pos) {
+    RowBatch b{0, pos, min(RB, rowEnd - pos)};
+    if constexpr (GSRC == kGradKernel) {
+      b.s = (pos >= src.end[0]) + (pos >= src.end[1]);
+      b.nr = min(b.nr, pick3(src.end, b.s) - pos);
+      if (b.s) b.row = pos - (b.s == 1 ? src.end[0] : src.end[1]);
+    }
+    return b;
+  };
+  auto row_of = [&](const RowBatch& b) { return (size_t)bh * (GSRC == kGradKernel ? pick3(src.len, b.s) : N) + b.row; };
+  auto fetch = [&](const RowBatch& b) {
+    const size_t row = row_of(b);
+    const T* qr = (GSRC == kGradKernel ? static_cast<const T*>(pick3(src.q, b.s)) : query) + row * C;
     if constexpr (GSRC == kGradF16) {
-      const int words = min(RB, rowEnd - rb) * MC / EPW;
-      const uint32_t* src = gw + (size_t)rb * MC / EPW;
+      const int words = b.nr * MC / EPW;
+      const uint32_t* gs = gw + (size_t)b.row * MC / EPW;
 #pragma unroll
       for (int t = 0; t < NL; ++t) {
         const int e = lane + 64 * t;
-        gpre[t] = e < words ? src[e] : 0u;
+        gpre[t] = e < words ? gs[e] : 0u;
       }
     } else {
-      // Branch-free: lanes past the batch re-read its last element (rb < rowEnd,
-      // so words >= MC >= 1) and are zeroed when the batch is staged.
-      const int words = min(RB, rowEnd - rb) * MC;
-      const float* gs = gkern + ((size_t)bh * N + rb) * MC;
-      const float* ks = kern + ((size_t)bh * N + rb) * MC;
+      // Branch-free: lanes past the batch re-read its last element (nr >= 1, so
+      // words >= MC >= 1) and are zeroed when the batch is staged.
+      const int words = b.nr * MC;
+      const float* gs = pick3(src.gk, b.s) + row * MC;
+      const float* ks = pick3(src.kv, b.s) + row * MC;
 #pragma unroll
       for (int t = 0; t < NL; ++t) {
         const int e = min(lane + 64 * t, words - 1);
@@ -782,161 +848,207 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, const float* __restrict__ g
       kwords = words;
     }
 #pragma unroll
-    for (int r = 0; r < RB; ++r) qpre[r] = (cval && rb + r < rowEnd) ? qb[(size_t)(rb + r) * C + c] : T{};
+    for (int i = 0; i < RB / RPW; ++i) {
+      const int r = RPW * i + hr;
+      qpre[i] = (cval && r < b.nr) ? qr[(size_t)r * C + c] : T{};
+    }
   };
   // The first batch's loads are in flight while the key tile is staged.
-  if (rowBeg < rowEnd) fetch(rowBeg);
-
-  for (int t = threadIdx.x; t < 64 * MC; t += blockDim.x) {
-    const int cl = t & 63, j = t >> 6;
-    const int cc = cb * 64 + cl;
-    ksm[j * 64 + cl] = cc < C ? to_acc(kb[(size_t)cc * MC + j]) * (kF16 ? 16777216.0f : 1.0f) : 0.0f;
+  RowBatch next{};
+  if (rowBeg < rowEnd) {
+    next = locate(rowBeg);
+    fetch(next);
   }
-  __syncthreads();
+
+  // Key tile (contiguous reads; the pitch of 65 spreads the stores over the banks): 16-bit
+  // keys as the step terms 1/2 - T(k), fp32 keys as values.
+  bool big = false;
+  for (int t = threadIdx.x; t < 64 * MC; t += blockDim.x) {
+    const int cl = t / MC, j = t - cl * MC;
+    const int cc = cb * 64 + cl;
+    const T kv = kb[(size_t)min(cc, C - 1) * MC + j];
+    float v;
+    if constexpr (k16) v = 0.5f - tmap16(kv.bits);
+    else v = to_acc(kv);
+    if constexpr (kTwo) big |= !(fabsf(v) < kStepKeyMax);
+    ksm[j * 65 + cl] = cc < C ? v : 0.0f;
+  }
+  bool fast = false;  // (workgroup-uniform)
+  if constexpr (kTwo) fast = !__syncthreads_or(big);
+  else __syncthreads();
+  const float pre = kTwo && fast ? kStepPre : 1.0f;
   float kreg[MC], dka[MC];
 #pragma unroll
   for (int j = 0; j < MC; ++j) {
-    kreg[j] = ksm[j * 64 + lane];
+    kreg[j] = ksm[j * 65 + ln] * pre;
     if (DK) dka[j] = 0.0f;
   }
   float hsum = 0.0f;  // lane j < MC: sum over this wave's rows of g[i][j]
-  // fp32 / bf16: the difference is scaled twice by 2^100 (a VGPR operand: an
-  // SGPR one would halve the issue rate) before the clamped half step.
-  float scl = 0x1p100f;
+  const uint32_t dcol = (uint32_t)(hr * C + c);  // the lane's element of a stored row (pair)
+  // (A VGPR operand: an SGPR one would halve the issue rate.)
+  float scl = kTwo && fast ? kStepFast : kStepSlow;
   asm volatile("" : "+v"(scl));
 
-  for (int rb = rowBeg; rb < rowEnd; rb += RB) {
-    const int nr = min(RB, rowEnd - rb);  // uniform
-    // Stage this batch: 2g as fp32, row-major [RB][MP] (exact for fp16 g; for the
-    // kernel gradient g = -s * gK * K, rounded once, then doubled exactly).
-    if constexpr (GSRC == kGradF16 && EPW == 2) {
+  auto batches = [&](auto fastc) {
+    for (int pos = rowBeg; pos < rowEnd;) {
+      const RowBatch cur = next;
+      const int nr = uniform(cur.nr);
+      pos += nr;
+      // Stage this batch: 2g as fp32, row-major [RB][MP] (exact for fp16 g; for the
+      // kernel gradient g = -s * gK * K, rounded once, then doubled exactly).
+      if constexpr (GSRC == kGradF16 && EPW == 2) {
 #pragma unroll
-      for (int t = 0; t < NL; ++t) {
-        const int e = 2 * (lane + 64 * t);
-        if (e < RB * MC) {
-          const int r0 = e / MC, j0 = e - r0 * MC;
-          const int r1 = (e + 1) / MC, j1 = e + 1 - r1 * MC;
-          float lo, hi;
-          if constexpr (kF16) {
-            lo = (float)__builtin_bit_cast(_Float16, (uint16_t)(gpre[t] & 0xffffu));
-            hi = (float)__builtin_bit_cast(_Float16, (uint16_t)(gpre[t] >> 16));
-          } else {  // bf16
-            lo = __builtin_bit_cast(float, gpre[t] << 16);
-            hi = __builtin_bit_cast(float, gpre[t] & 0xffff0000u);
-          }
-          gsm[r0 * MP + j0] = 2.0f * lo;
-          gsm[r1 * MP + j1] = 2.0f * hi;
-        }
-      }
-    } else if constexpr (GSRC == kGradF16) {  // fp32: one element per word
-#pragma unroll
-      for (int t = 0; t < NL; ++t) {
-        const int e = lane + 64 * t;
-        if (e < RB * MC) {
-          const int r = e / MC, j = e - r * MC;
-          gsm[r * MP + j] = 2.0f * __builtin_bit_cast(float, gpre[t]);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < NL; ++t) {
-        const int e = lane + 64 * t;
-        if (e < RB * MC) {
-          const int r = e / MC, j = e - r * MC;
-          const float v = (gscale2 * __builtin_bit_cast(float, gpre[t])) * kpre[t];
-          gsm[r * MP + j] = e < kwords ? v : 0.0f;
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < RB; ++r) qsm[r * 64 + lane] = to_acc(qpre[r]) * (kF16 ? 16777216.0f : 1.0f);
-    wave_sync();
-    // Row sums (lane r) for grad_query and column sums (lane j) for grad_key.
-    // Rows past nr are zero in the batch. All reads of a sum are issued before
-    // the additions, so no chain of dependent LDS round trips.
-    if (DQ) {
-      const float4* rowp = reinterpret_cast<const float4*>(gsm + min(lane, RB - 1) * MP);
-      float4 v[MP / 4];
-#pragma unroll
-      for (int jq = 0; jq < MP / 4; ++jq) v[jq] = rowp[jq];
-      float sum = 0.0f;
-#pragma unroll
-      for (int jq = 0; jq < MP / 4; ++jq) {
-        const float e[4] = {v[jq].x, v[jq].y, v[jq].z, v[jq].w};
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          if (jq * 4 + t < MC) sum += e[t];
-      }
-      if (lane < RB) gneg[lane] = -0.5f * sum;
-    }
-    if (DK) {
-      float hv[RB];
-#pragma unroll
-      for (int r = 0; r < RB; ++r) hv[r] = gsm[r * MP + min(lane, MC - 1)];
-#pragma unroll
-      for (int r = 0; r < RB; ++r) hsum += hv[r];
-    }
-    wave_sync();
-    if (rb + RB < rowEnd) fetch(rb + RB);
-
-    // Row loop, software-pipelined two broadcast reads ahead (LDS latency under
-    // load exceeds one column group's VALU time); the next row's query value,
-    // initial sum and first two grad groups are read during the current row's
-    // last groups. The scheduling barriers keep the compiler from computing
-    // every column's step up front (MC more registers).
-    constexpr int NQ = MP / 4;
-    static_assert(NQ >= 2 && NQ % 2 == 0, "two groups in flight, slots aligned at every row start");
-    float qn = qsm[lane];
-    float accn = DQ ? gneg[0] : 0.0f;
-    float4 gq[2] = {reinterpret_cast<const float4*>(gsm)[0], reinterpret_cast<const float4*>(gsm)[1]};
-#pragma unroll 1
-    for (int r = 0; r < nr; ++r) {
-      const float4* g4 = reinterpret_cast<const float4*>(gsm + r * MP);
-      const float4* g4n = reinterpret_cast<const float4*>(gsm + min(r + 1, RB - 1) * MP);
-      const float qv = qn;
-      // grad_query of the row as four independent partial sums (columns j = t
-      // mod 4), combined once at the end: a single chain of MC dependent FMAs
-      // would stall a wave on every column.
-      float acc[4] = {accn, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int jq = 0; jq < NQ; ++jq) {
-        const float4 gv = gq[jq & 1];
-        if (jq + 2 < NQ) gq[jq & 1] = g4[jq + 2];
-        else gq[jq & 1] = g4n[jq + 2 - NQ];
-        if (jq == NQ - 1) {
-          qn = qsm[min(r + 1, RB - 1) * 64 + lane];
-          if (DQ) accn = gneg[min(r + 1, RB - 1)];
-        }
-        const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int j = jq * 4 + t;
-          if (j < MC) {
-            float y;
+        for (int t = 0; t < NL; ++t) {
+          const int e = 2 * (lane + 64 * t);
+          if (e < RB * MC) {
+            const int r0 = e / MC, j0 = e - r0 * MC;
+            const int r1 = (e + 1) / MC, j1 = e + 1 - r1 * MC;
+            float lo, hi;
             if constexpr (kF16) {
-              y = half_step(qv - kreg[j]);
-            } else {
-              const float e = (qv - kreg[j]) * scl;
-              y = __builtin_amdgcn_fmed3f(__builtin_fmaf(e, scl, 0.5f), 0.0f, 1.0f);
+              lo = (float)__builtin_bit_cast(_Float16, (uint16_t)(gpre[t] & 0xffffu));
+              hi = (float)__builtin_bit_cast(_Float16, (uint16_t)(gpre[t] >> 16));
+            } else {  // bf16
+              lo = __builtin_bit_cast(float, gpre[t] << 16);
+              hi = __builtin_bit_cast(float, gpre[t] & 0xffff0000u);
             }
-            if (DQ) acc[t] = fmaf(gg[t], y, acc[t]);
-            if (DK) {
-              dka[j] = fmaf(gg[t], y, dka[j]);
-              asm volatile("" : "+v"(dka[j]));  // update in place, not after the row
-            }
+            gsm[r0 * MP + j0] = 2.0f * lo;
+            gsm[r1 * MP + j1] = 2.0f * hi;
           }
         }
-        __builtin_amdgcn_sched_barrier(0);
+      } else if constexpr (GSRC == kGradF16) {  // fp32: one element per word
+#pragma unroll
+        for (int t = 0; t < NL; ++t) {
+          const int e = lane + 64 * t;
+          if (e < RB * MC) {
+            const int r = e / MC, j = e - r * MC;
+            gsm[r * MP + j] = 2.0f * __builtin_bit_cast(float, gpre[t]);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < NL; ++t) {
+          const int e = lane + 64 * t;
+          if (e < RB * MC) {
+            const int r = e / MC, j = e - r * MC;
+            const float v = (gscale2 * __builtin_bit_cast(float, gpre[t])) * kpre[t];
+            gsm[r * MP + j] = e < kwords ? v : 0.0f;
+          }
+        }
       }
+#pragma unroll
+      for (int i = 0; i < RB / RPW; ++i) {
+        if constexpr (k16) qsm[i * 64 + lane] = tmap16(qpre[i].bits);
+        else qsm[i * 64 + lane] = to_acc(qpre[i]) * pre;
+      }
+      wave_sync();
+      // Row sums (lane r) for grad_query and column sums (lane j) for grad_key.
+      // Rows past nr are zero in the batch. All reads of a sum are issued before
+      // the additions, so no chain of dependent LDS round trips.
       if (DQ) {
-        float total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        // Materialise the sum here: sunk into the store's branch, the
-        // accumulation would keep every column's step value live.
-        asm volatile("" : "+v"(total));
-        if (cval) dq[((size_t)bh * N + rb + r) * C + c] = from_acc<T>(total);
+        const float4* rowp = reinterpret_cast<const float4*>(gsm + min(lane, RB - 1) * MP);
+        // (Half the row at a time: a whole row's registers would spill some of the columns'.)
+        constexpr int HQ = MP / 8;
+        float sum = 0.0f;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float4 v[HQ];
+#pragma unroll
+          for (int jq = 0; jq < HQ; ++jq) v[jq] = rowp[h * HQ + jq];
+#pragma unroll
+          for (int jq = 0; jq < HQ; ++jq) {
+            const float e[4] = {v[jq].x, v[jq].y, v[jq].z, v[jq].w};
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+              if ((h * HQ + jq) * 4 + t < MC) sum += e[t];
+          }
+          asm volatile("" : "+v"(sum)::"memory");
+        }
+        if (lane < RB) gneg[lane] = -0.5f * sum;
       }
+      if (DK) {
+        float hv[RB];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) hv[r] = gsm[r * MP + min(lane, MC - 1)];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) hsum += hv[r];
+      }
+      wave_sync();
+      if (pos < rowEnd) {
+        next = locate(pos);
+        fetch(next);
+      }
+      T* dqr = (GSRC == kGradKernel ? static_cast<T*>(pick3(src.dq, cur.s)) : dq) + row_of(cur) * C;
+
+      // Row loop, software-pipelined two broadcast reads ahead (LDS latency under
+      // load exceeds one column group's VALU time); the next row's query value,
+      // initial sum and first two grad groups are read during the current row's
+      // last groups. The scheduling barriers keep the compiler from computing
+      // every column's step up front (MC more registers).
+      constexpr int NQ = MP / 4;
+      static_assert(NQ >= 2 && NQ % 2 == 0, "two groups in flight, slots aligned at every row start");
+      // (Row pair i of a batch is rows RPW i + hr; rows past nr are zero there.)
+      const float* gh = gsm + hr * MP;
+      float qn = qsm[lane];
+      float accn = DQ ? gneg[hr] : 0.0f;
+      float4 gq[2] = {reinterpret_cast<const float4*>(gh)[0], reinterpret_cast<const float4*>(gh)[1]};
+#pragma unroll 1
+      for (int i = 0; i * RPW < nr; ++i) {
+        const int in = min(i + 1, RB / RPW - 1);
+        const float4* g4 = reinterpret_cast<const float4*>(gh + RPW * i * MP);
+        const float4* g4n = reinterpret_cast<const float4*>(gh + RPW * in * MP);
+        const float qv = qn;
+        // grad_query of the row as four independent partial sums (columns j = t
+        // mod 4), combined once at the end: a single chain of MC dependent FMAs
+        // would stall a wave on every column.
+        float acc[4] = {accn, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int jq = 0; jq < NQ; ++jq) {
+          const float4 gv = gq[jq & 1];
+          if (jq + 2 < NQ) gq[jq & 1] = g4[jq + 2];
+          else gq[jq & 1] = g4n[jq + 2 - NQ];
+          if (jq == NQ - 1) {
+            qn = qsm[in * 64 + lane];
+            if (DQ) accn = gneg[RPW * in + hr];
+          }
+          const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const int j = jq * 4 + t;
+            if (j < MC) {
+              float y;
+              if constexpr (k16) {
+                y = __builtin_amdgcn_fmed3f(qv + kreg[j], 0.0f, 1.0f);  // one clamped add
+              } else if constexpr (decltype(fastc)::value) {
+                y = __builtin_amdgcn_fmed3f(__builtin_fmaf(qv - kreg[j], scl, 0.5f), 0.0f, 1.0f);
+              } else {
+                const float e = (qv - kreg[j]) * scl;
+                y = __builtin_amdgcn_fmed3f(__builtin_fmaf(e, scl, 0.5f), 0.0f, 1.0f);
+              }
+              if (DQ) acc[t] = fmaf(gg[t], y, acc[t]);
+              if (DK) {
+                dka[j] = fmaf(gg[t], y, dka[j]);
+                asm volatile("" : "+v"(dka[j]));  // update in place, not after the row
+              }
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (DQ) {
+          float total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+          // Materialise the sum here: sunk into the store's branch, the
+          // accumulation would keep every column's step value live.
+          asm volatile("" : "+v"(total));
+          if (cval && (RPW == 1 || RPW * i + hr < nr)) (dqr + (size_t)(RPW * i) * C)[dcol] = from_acc<T>(total);
+        }
+      }
+      wave_sync();
     }
-    wave_sync();
+  };
+  if constexpr (kTwo) {
+    if (fast) batches(std::true_type{});
+    else batches(std::false_type{});
+  } else {
+    batches(std::false_type{});
   }
 
   if (DK) {
@@ -944,9 +1056,20 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, const float* __restrict__ g
     if (lane < MC) hsm[lane] = 0.5f * hsum;
     wave_sync();
 #pragma unroll
-    for (int j = 0; j < MC; ++j) dka[j] = hsm[j] - dka[j];
-    bcast_reduce_dk<MC>(dka, reinterpret_cast<float*>(smem), W, wave, lane,
-                        partial + ((size_t)slice * nx + x) * 64 * MC);
+    for (int j = 0; j < MC; ++j) {
+      if constexpr (RPW == 2) dka[j] += __shfl_xor(dka[j], 32);
+      dka[j] = hsm[j] - dka[j];
+    }
+    // The slice's only workgroup stores grad_key itself; else the reduction kernel sums
+    // the workgroups' partials ([MC][64]) in order.
+    const bool only = nx == 1;
+    float* pout = partial + ((size_t)slice * nx + x) * 64 * MC;
+    T* dkb = dk + ((size_t)bh * C + cb * 64) * MC;
+    const int cn = C - cb * 64;
+    bcast_reduce_dk<MC>(dka, reinterpret_cast<float*>(smem), W, wave, lane, only, [&](int j, int cl, float v) {
+      if (!only) pout[j * 64 + cl] = v;
+      else if (cl < cn) dkb[cl * MC + j] = from_acc<T>(v);
+    });
   }
 }
 
@@ -956,19 +1079,17 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, const float* __restrict__ g
 //
 // A workgroup is RG row groups of CB waves; wave (g, b) of a group takes the
 // 32 columns [32b, 32b + 32) of every row batch (RB rows) of its group, with
-// its columns' key values and grad_key sums in registers, as the fp16 kernel
-// above does for all columns. A row's grad_query is the sum of the CB waves'
+// its columns' key values and grad_key sums in registers, as the kernel above does
+// for all columns. A row's grad_query is the sum of the CB waves'
 // column-block partials: each wave leaves its partials in LDS (double-buffered
 // by batch parity), and after one workgroup barrier per batch each wave of the
 // group sums RB/CB of the batch's rows in column-block order (deterministic).
 // grad_key: the RG groups' sums in group order, then the workgroup partials
 // summed over the slice by the reduction kernel.
 //
-// Step y = (sgn(q - k) + 1)/2 at the full VALU rate: fp16 operands pre-scaled
-// by 2^24 (d = 0 or |d| >= 1, y = clamp(d/2 + 1/2)); bf16/fp32 by scaling the
-// difference twice by 2^100 (every nonzero fp32 difference is >= 2^-149, so
-// |d| * 2^200 >= 2^51; overflow to +-inf clamps correctly), five instructions
-// per triple instead of four.
+// Step y = (sgn(q - k) + 1)/2 at the full VALU rate: 16-bit operands through their
+// ordered patterns (tmap16), one clamped add; fp32 in two or three instructions
+// (kStepFast, kStepSlow).
 // ---------------------------------------------------------------------------
 constexpr int kMbMC = 32;  // columns per wave
 constexpr int kMbRB = 8;   // rows per batch
@@ -977,7 +1098,7 @@ template <typename T, int CB, bool DQ, bool DK, int GSRC = kGradF16>
 __global__ void __launch_bounds__(1024)
 laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, const T* __restrict__ key,
                       T* __restrict__ dq, float* __restrict__ partial, int N, int C, int rowsPerWG, int Mt,
-                      const float* __restrict__ gkern, const float* __restrict__ kern, float gscale) {
+                      RowSources src, float gscale) {
   // M = CB * 32 columns in registers and LDS; the tensors have Mt <= M columns (the
   // last block is partial when Mt is not a multiple of 32: its columns from Mt on
   // have zero grad and key, so they add nothing and are not stored).
@@ -985,9 +1106,9 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
   constexpr int MP = MC;                       // LDS row pitch of a staged batch (floats)
   // 16-bit inputs take the ordered-pattern step (tmap16): y = clamp(T(q) + (1/2 - T(k))).
   constexpr bool k16 = std::is_same<T, f16s>::value || std::is_same<T, bf16s>::value;
+  constexpr bool kTwo = two_step_loops<T, DQ, DK, GSRC>();
   // Grad elements per fetched 32-bit word: 2 for 16-bit grads, 1 for fp32 grads and
   // for the kernel-gradient source (fp32 gK and K, g = -s * gK * K formed at staging).
-  static_assert(GSRC == kGradF16 || std::is_same<T, f16s>::value, "kernel-gradient source: fp16 only");
   constexpr int EPW = GSRC == kGradKernel ? 1 : (4 / (int)sizeof(T) > 0 ? 4 / (int)sizeof(T) : 1);
   constexpr int GW = RB * MC / EPW;            // grad words of a batch (this wave's columns)
   constexpr int NL = (GW + 63) / 64;           // words per lane
@@ -1001,9 +1122,9 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
   const int c = chb * 64 + lane;
   const bool cval = c < C;
   const int cq = min(c, C - 1);
-  const int r0wg = x * rowsPerWG;
-  const int rowsWG = max(0, min(N, r0wg + rowsPerWG) - r0wg);
-  const int nb = (rowsWG + RB - 1) / RB;        // batches of the workgroup
+  // Batches of RB rows, each of one row set (the sets' ends in src count batches).
+  const int b0 = x * (rowsPerWG / RB);
+  const int nb = max(0, min((GSRC == kGradKernel ? src.end[2] : (N + RB - 1) / RB) - b0, rowsPerWG / RB));
   const int rounds = (nb + RG - 1) / RG;        // batch t goes to group t % RG
 
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1014,7 +1135,18 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
   float* gneg = gsm + RB * MP;                                      // [RB] -sum_j g,
   float* qsm = gneg + RB;                                           // [RB][64] query values
 
-  const T* qb = query + (size_t)bh * N * C;
+  auto locate = [&](int t) {
+    RowBatch b{0, (b0 + t) * RB, 0};
+    int len = N;
+    if constexpr (GSRC == kGradKernel) {
+      b.s = (b0 + t >= src.end[0]) + (b0 + t >= src.end[1]);
+      if (b.s) b.row -= RB * (b.s == 1 ? src.end[0] : src.end[1]);
+      len = pick3(src.len, b.s);
+    }
+    b.nr = min(RB, len - b.row);
+    return b;
+  };
+  auto row_of = [&](const RowBatch& b) { return (size_t)bh * (GSRC == kGradKernel ? pick3(src.len, b.s) : N) + b.row; };
   const T* kb = key + (size_t)bh * C * Mt;
 
   // Next batch of this group: this wave's 32 columns of RB rows (clamped to the
@@ -1025,20 +1157,21 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
   T qpre[RB];
   int fnr = 0;
   auto fetch = [&](int t) {
-    const int rb = r0wg + t * RB;
-    const int nr = min(RB, r0wg + rowsWG - rb);
+    const RowBatch b = locate(t);
+    const int nr = b.nr;
+    const size_t row = row_of(b);
 #pragma unroll
     for (int s = 0; s < NL; ++s) {
       const int w = lane + 64 * s;               // word of the batch block
       const int r = min(w / (MC / EPW), nr - 1), jw = w - (w / (MC / EPW)) * (MC / EPW);
       const int col = cbk * MC + jw * EPW;
       if constexpr (GSRC == kGradKernel) {
-        const size_t o = ((size_t)bh * N + rb + r) * Mt + min(col, Mt - 1);
-        gpre[s] = col < Mt ? __builtin_bit_cast(uint32_t, gkern[o]) : 0u;
-        kpre[s] = col < Mt ? kern[o] : 0.0f;
+        const size_t o = (row + r) * Mt + min(col, Mt - 1);
+        gpre[s] = col < Mt ? __builtin_bit_cast(uint32_t, pick3(src.gk, b.s)[o]) : 0u;
+        kpre[s] = col < Mt ? pick3(src.kv, b.s)[o] : 0.0f;
         continue;
       }
-      const T* rowp = gout + ((size_t)bh * N + rb + r) * Mt;
+      const T* rowp = gout + (row + r) * Mt;
       if constexpr (EPW == 2) {
         if (Mt & 1) {  // odd row length: rows do not start on 4-byte words, two 16-bit loads
           const uint32_t lo = col < Mt ? rowp[min(col, Mt - 1)].bits : 0u;
@@ -1051,7 +1184,8 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
       gpre[s] = col < Mt ? *reinterpret_cast<const uint32_t*>(rowp + min(col, Mt - EPW)) : 0u;
     }
 #pragma unroll
-    for (int r = 0; r < RB; ++r) qpre[r] = qb[(size_t)min(rb + r, rb + nr - 1) * C + cq];
+    for (int r = 0; r < RB; ++r)
+      qpre[r] = (GSRC == kGradKernel ? static_cast<const T*>(pick3(src.q, b.s)) : query)[(row + min(r, nr - 1)) * C + cq];
     fnr = nr;
   };
   int t0 = grp;  // this group's first batch
@@ -1059,6 +1193,7 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
 
   // Key tile (global [C][M], coalesced over j): 16-bit keys as the step terms
   // 1/2 - T(k) (see tmap16), fp32 keys as values. Columns past Mt have zero grad.
+  bool huge = false;
   for (int t = threadIdx.x; t < 64 * M; t += blockDim.x) {
     const int cl = t / M, j = t - cl * M;
     const int cc = chb * 64 + cl;
@@ -1066,139 +1201,163 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
     const T kv = kb[(size_t)min(cc, C - 1) * Mt + min(j, Mt - 1)];
     if constexpr (k16)
       big[j * 64 + cl] = in ? 0.5f - tmap16(kv.bits) : 0.0f;
-    else
+    else {
+      if constexpr (kTwo) huge |= !(fabsf(to_acc(kv)) < kStepKeyMax);
       big[j * 64 + cl] = in ? to_acc(kv) : 0.0f;
+    }
   }
-  __syncthreads();
+  bool fast = false;  // (workgroup-uniform)
+  if constexpr (kTwo) fast = !__syncthreads_or(huge);
+  else __syncthreads();
+  const float pre = kTwo && fast ? kStepPre : 1.0f;
   float kreg[MC], dka[MC];
 #pragma unroll
   for (int j = 0; j < MC; ++j) {
-    kreg[j] = big[(cbk * MC + j) * 64 + lane];
+    kreg[j] = big[(cbk * MC + j) * 64 + lane] * pre;
     if (DK) dka[j] = 0.0f;
   }
   __syncthreads();  // the key tile's LDS becomes the partial buffers
-  float scl = 0x1p100f;
+  float scl = kTwo && fast ? kStepFast : kStepSlow;
   asm volatile("" : "+v"(scl));  // VGPR operand: an SGPR one would halve the issue rate
   float hsum = 0.0f;  // lane j < MC: sum over this wave's rows of 2 g[i][j]
 
-  for (int round = 0; round < rounds; ++round) {
-    const int t = round * RG + grp;
-    const bool have = t < nb;                          // uniform per wave
-    const int nr = have ? fnr : 0;
-    float* dqp = big + ((round & 1) * W + wave) * RB * 64;  // this wave's partials of this batch
-    if (have) {
-      // Stage: 2g as fp32 [RB][MP], rows past nr zero.
-#pragma unroll
-      for (int s = 0; s < NL; ++s) {
-        const int w = lane + 64 * s;
-        const int r = w / (MC / EPW), jw = w - r * (MC / EPW);
-        const bool ok = r < nr;
-        if constexpr (EPW == 2) {
-          const float lo = std::is_same<T, f16s>::value
-                               ? (float)__builtin_bit_cast(_Float16, (uint16_t)(gpre[s] & 0xffffu))
-                               : __builtin_bit_cast(float, gpre[s] << 16);
-          const float hi = std::is_same<T, f16s>::value
-                               ? (float)__builtin_bit_cast(_Float16, (uint16_t)(gpre[s] >> 16))
-                               : __builtin_bit_cast(float, gpre[s] & 0xffff0000u);
-          gsm[r * MP + 2 * jw] = ok ? 2.0f * lo : 0.0f;
-          gsm[r * MP + 2 * jw + 1] = ok ? 2.0f * hi : 0.0f;
-        } else if constexpr (GSRC == kGradKernel) {
-          gsm[r * MP + jw] = ok ? (gscale2 * __builtin_bit_cast(float, gpre[s])) * kpre[s] : 0.0f;
-        } else {
-          gsm[r * MP + jw] = ok ? 2.0f * __builtin_bit_cast(float, gpre[s]) : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < RB; ++r) {
-        if constexpr (k16)
-          qsm[r * 64 + lane] = tmap16(qpre[r].bits);
-        else
-          qsm[r * 64 + lane] = to_acc(qpre[r]);
-      }
-      wave_sync();
-      if (DQ) {
-        const float4* rowp = reinterpret_cast<const float4*>(gsm + min(lane, RB - 1) * MP);
-        float4 v[MP / 4];
-#pragma unroll
-        for (int jq = 0; jq < MP / 4; ++jq) v[jq] = rowp[jq];
-        float sum = 0.0f;
-#pragma unroll
-        for (int jq = 0; jq < MP / 4; ++jq) sum += (v[jq].x + v[jq].y) + (v[jq].z + v[jq].w);
-        if (lane < RB) gneg[lane] = -0.5f * sum;
-      }
-      if (DK) {
-        float hv[RB];
-#pragma unroll
-        for (int r = 0; r < RB; ++r) hv[r] = gsm[r * MP + min(lane, MC - 1)];
-#pragma unroll
-        for (int r = 0; r < RB; ++r) hsum += hv[r];
-      }
-      wave_sync();
-      if (t + RG < nb) fetch(t + RG);
-
-      // Row loop as in the fp16 kernel: grad values two 16-byte groups ahead,
-      // four partial sums per row, grad_key sums updated in place.
-      constexpr int NQ = MP / 4;
-      float qn = qsm[lane];
-      float accn = DQ ? gneg[0] : 0.0f;
-      float4 gq[2] = {reinterpret_cast<const float4*>(gsm)[0], reinterpret_cast<const float4*>(gsm)[1]};
-#pragma unroll 1
-      for (int r = 0; r < nr; ++r) {
-        const float4* g4 = reinterpret_cast<const float4*>(gsm + r * MP);
-        const float4* g4n = reinterpret_cast<const float4*>(gsm + min(r + 1, RB - 1) * MP);
-        const float qv = qn;
-        float acc[4] = {accn, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int jq = 0; jq < NQ; ++jq) {
-          const float4 gv = gq[jq & 1];
-          if (jq + 2 < NQ) gq[jq & 1] = g4[jq + 2];
-          else gq[jq & 1] = g4n[jq + 2 - NQ];
-          if (jq == NQ - 1) {
-            qn = qsm[min(r + 1, RB - 1) * 64 + lane];
-            if (DQ) accn = gneg[min(r + 1, RB - 1)];
-          }
-          const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int j = jq * 4 + u;
-            float y;
-            if constexpr (k16) {
-              y = __builtin_amdgcn_fmed3f(qv + kreg[j], 0.0f, 1.0f);  // one clamped add
-            } else {
-              const float e = (qv - kreg[j]) * scl;
-              y = __builtin_amdgcn_fmed3f(__builtin_fmaf(e, scl, 0.5f), 0.0f, 1.0f);
-            }
-            if (DQ) acc[u] = fmaf(gg[u], y, acc[u]);
-            if (DK) {
-              dka[j] = fmaf(gg[u], y, dka[j]);
-              asm volatile("" : "+v"(dka[j]));  // update in place, not after the row
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (DQ) {
-          float total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-          asm volatile("" : "+v"(total));
-          dqp[r * 64 + lane] = total;
-        }
-      }
-    }
-    if (DQ) {
-      // Every wave of the workgroup has written this batch's partials (and is
-      // done reading the partials of two batches ago, in the other buffer).
-      __syncthreads();
+  auto batches = [&](auto fastc) {
+    for (int round = 0; round < rounds; ++round) {
+      const int t = round * RG + grp;
+      const bool have = t < nb;                          // uniform per wave
+      const int nr = have ? fnr : 0;
+      float* dqp = big + ((round & 1) * W + wave) * RB * 64;  // this wave's partials of this batch
       if (have) {
-        const int rb = r0wg + t * RB;
-        const float* gp = big + ((round & 1) * W + grp * CB) * RB * 64;  // the group's CB waves
-        for (int r = cbk; r < nr; r += CB) {
-          float sv = 0.0f;
+        // Stage: 2g as fp32 [RB][MP], rows past nr zero.
 #pragma unroll
-          for (int b = 0; b < CB; ++b) sv += gp[(b * RB + r) * 64 + lane];
-          if (cval) dq[((size_t)bh * N + rb + r) * C + c] = from_acc<T>(sv);
+        for (int s = 0; s < NL; ++s) {
+          const int w = lane + 64 * s;
+          const int r = w / (MC / EPW), jw = w - r * (MC / EPW);
+          const bool ok = r < nr;
+          if constexpr (EPW == 2) {
+            const float lo = std::is_same<T, f16s>::value
+                                 ? (float)__builtin_bit_cast(_Float16, (uint16_t)(gpre[s] & 0xffffu))
+                                 : __builtin_bit_cast(float, gpre[s] << 16);
+            const float hi = std::is_same<T, f16s>::value
+                                 ? (float)__builtin_bit_cast(_Float16, (uint16_t)(gpre[s] >> 16))
+                                 : __builtin_bit_cast(float, gpre[s] & 0xffff0000u);
+            gsm[r * MP + 2 * jw] = ok ? 2.0f * lo : 0.0f;
+            gsm[r * MP + 2 * jw + 1] = ok ? 2.0f * hi : 0.0f;
+          } else if constexpr (GSRC == kGradKernel) {
+            gsm[r * MP + jw] = ok ? (gscale2 * __builtin_bit_cast(float, gpre[s])) * kpre[s] : 0.0f;
+          } else {
+            gsm[r * MP + jw] = ok ? 2.0f * __builtin_bit_cast(float, gpre[s]) : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+          if constexpr (k16)
+            qsm[r * 64 + lane] = tmap16(qpre[r].bits);
+          else
+            qsm[r * 64 + lane] = to_acc(qpre[r]) * pre;
+        }
+        wave_sync();
+        if (DQ) {
+          const float4* rowp = reinterpret_cast<const float4*>(gsm + min(lane, RB - 1) * MP);
+          float4 v[MP / 4];
+#pragma unroll
+          for (int jq = 0; jq < MP / 4; ++jq) v[jq] = rowp[jq];
+          float sum = 0.0f;
+#pragma unroll
+          for (int jq = 0; jq < MP / 4; ++jq) sum += (v[jq].x + v[jq].y) + (v[jq].z + v[jq].w);
+          if (lane < RB) gneg[lane] = -0.5f * sum;
+        }
+        if (DK) {
+          float hv[RB];
+#pragma unroll
+          for (int r = 0; r < RB; ++r) hv[r] = gsm[r * MP + min(lane, MC - 1)];
+#pragma unroll
+          for (int r = 0; r < RB; ++r) hsum += hv[r];
+        }
+        wave_sync();
+        if (t + RG < nb) fetch(t + RG);
+
+        // Row loop as in the register-column kernel above (grad values two 16-byte groups
+        // ahead, four partial sums per row, grad_key sums updated in place), unrolled over
+        // the whole batch so that every LDS address is an immediate (rows past nr have zero
+        // grad and are not stored). That leaves the registers to fit: a spilled one is
+        // reloaded behind the next batch's loads, whose latency it then waits for. bf16,
+        // 128 slices, N = 4096, M = 256, C = 64, both gradients: 798 -> 660 us (1.3 ns per
+        // VALU instruction and SIMD, 1.0 to 1.35 being the rate of four waves of the loop's
+        // adds and FMAs alone); three or four groups ahead spill 6 to 12 registers and take
+        // 750 to 800 us; half waves on 16 columns x 2 channels each, which halve the LDS
+        // reads, spill 2 and take 699 us, and gain 1 to 3 % where only one gradient is asked.
+        constexpr int NQ = MP / 4, NG = RB * NQ, LA = 2;
+        const float4* g4 = reinterpret_cast<const float4*>(gsm);
+        float qn = qsm[lane];
+        float accn = DQ ? gneg[0] : 0.0f;
+        float4 gq[LA];
+#pragma unroll
+        for (int u = 0; u < LA; ++u) gq[u] = g4[u];
+        unrolled<RB>([&](auto rc) {
+          constexpr int r = rc.value;
+          const float qv = qn;
+          float acc[4] = {accn, 0.0f, 0.0f, 0.0f};
+          unrolled<NQ>([&](auto jc) {
+            constexpr int jq = jc.value, at = r * NQ + jq;
+            const float4 gv = gq[at % LA];
+            if constexpr (at + LA < NG) gq[at % LA] = g4[at + LA];
+            if constexpr (jq == NQ - 1 && r + 1 < RB) {
+              qn = qsm[(r + 1) * 64 + lane];
+              if (DQ) accn = gneg[r + 1];
+            }
+            const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int j = jq * 4 + u;
+              float y;
+              if constexpr (k16) {
+                y = __builtin_amdgcn_fmed3f(qv + kreg[j], 0.0f, 1.0f);  // one clamped add
+              } else if constexpr (decltype(fastc)::value) {
+                y = __builtin_amdgcn_fmed3f(__builtin_fmaf(qv - kreg[j], scl, 0.5f), 0.0f, 1.0f);
+              } else {
+                const float e = (qv - kreg[j]) * scl;
+                y = __builtin_amdgcn_fmed3f(__builtin_fmaf(e, scl, 0.5f), 0.0f, 1.0f);
+              }
+              if (DQ) acc[u] = fmaf(gg[u], y, acc[u]);
+              if (DK) {
+                dka[j] = fmaf(gg[u], y, dka[j]);
+                asm volatile("" : "+v"(dka[j]));  // update in place, not after the row
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          });
+          if (DQ) {
+            float total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            asm volatile("" : "+v"(total));
+            dqp[r * 64 + lane] = total;
+          }
+        });
+      }
+      if (DQ) {
+        // Every wave of the workgroup has written this batch's partials (and is
+        // done reading the partials of two batches ago, in the other buffer).
+        __syncthreads();
+        if (have) {
+          const RowBatch b = locate(t);
+          T* dqr = (GSRC == kGradKernel ? static_cast<T*>(pick3(src.dq, b.s)) : dq) + row_of(b) * C;
+          const float* gp = big + ((round & 1) * W + grp * CB) * RB * 64;  // the group's CB waves
+          for (int r = cbk; r < nr; r += CB) {
+            float sv = 0.0f;
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) sv += gp[(cb * RB + r) * 64 + lane];
+            if (cval) dqr[(size_t)r * C + c] = from_acc<T>(sv);
+          }
         }
       }
+      if (have) wave_sync();
     }
-    if (have) wave_sync();
+  };
+  if constexpr (kTwo) {
+    if (fast) batches(std::true_type{});
+    else batches(std::false_type{});
+  } else {
+    batches(std::false_type{});
   }
 
   if (DK) {
@@ -1579,58 +1738,56 @@ BcPlan plan_bcast(const Dims& d, bool dkey) {
   p.nx = ceil_div((int)wps, W);
   p.rowsPerWave = round_up(ceil_div(N, p.nx * W), 2);
   const int mp = bcast_pitch((int)d.M);
-  p.lds = ((size_t)d.M * 64 + (size_t)W * (kBcRB * mp + kBcRB + mp + kBcRB * 64)) * 4;
-  if (dkey) p.lds = std::max(p.lds, (size_t)std::min(W, kBcBufs) * d.M * 64 * 4);
+  const int rpw = d.C <= 32 ? 2 : 1;
+  p.lds = ((size_t)bcast_key_floats((int)d.M) + (size_t)W * (kBcRB * mp + kBcRB + mp + kBcRB / rpw * 64)) * 4;
+  if (dkey) p.lds = std::max(p.lds, (size_t)std::min(W, kBcBufs) * bcast_key_floats((int)d.M) * 4);
   p.partialElems = dkey ? (size_t)slices * p.nx * 64 * (size_t)d.M : 0;
   return p;
 }
 
 // Kernel-gradient source of the backward (LaplacianFormer's K = exp(-s * dist)).
 struct KernGrad {
-  const float* gk = nullptr;
-  const float* kv = nullptr;
+  RowSources src = {};
   float scale = 0.0f;
 };
 
-template <typename T, int MC, bool DQ, bool DK, int GSRC = kGradF16>
-int launch_bcast_bwd_mc(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
-                        const BcPlan& p, hipStream_t st, KernGrad kg = {}) {
+template <typename T, int MC, bool DQ, bool DK, int GSRC, int RPW>
+int launch_bcast_bwd_rpw(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
+                         const BcPlan& p, hipStream_t st, const KernGrad& kg) {
   dim3 grid(p.nx, p.ncb, (unsigned)d.BH());
-  hipLaunchKernelGGL((laplace_bwd_bcast_kernel<T, MC, DQ, DK, GSRC>), grid, dim3(64 * p.W), p.lds, st,
-                     static_cast<const T*>(g), kg.gk, kg.kv, kg.scale, static_cast<const T*>(q),
+  hipLaunchKernelGGL((laplace_bwd_bcast_kernel<T, MC, DQ, DK, GSRC, RPW>), grid, dim3(64 * p.W), p.lds, st,
+                     static_cast<const T*>(g), kg.src, kg.scale, static_cast<const T*>(q),
                      static_cast<const T*>(k), static_cast<T*>(dq), static_cast<T*>(dk),
                      static_cast<float*>(ws), (int)d.N, (int)d.C, p.rowsPerWave);
-  int s = check_launch("laplace backward");
-  if (s || !DK) return s;
+  return check_launch("laplace backward");
+}
+
+template <typename T, int MC, bool DQ, bool DK, int GSRC>
+int launch_bcast_bwd_mc(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
+                        const BcPlan& p, hipStream_t st, const KernGrad& kg) {
+  int s = d.C <= 32 ? launch_bcast_bwd_rpw<T, MC, DQ, DK, GSRC, 2>(g, q, k, dq, dk, ws, d, p, st, kg)
+                    : launch_bcast_bwd_rpw<T, MC, DQ, DK, GSRC, 1>(g, q, k, dq, dk, ws, d, p, st, kg);
+  if (s || !DK || p.nx == 1) return s;
   dim3 rgrid(ceil_div(64 * MC, 256), p.ncb, (unsigned)d.BH());
   hipLaunchKernelGGL(laplace_dk_reduce_cm_kernel<T>, rgrid, dim3(256), 0, st, static_cast<const float*>(ws),
                      static_cast<T*>(dk), p.nx, MC, (int)d.C);
   return check_launch("laplace backward_key reduction");
 }
 
-template <typename T, bool DQ, bool DK, int GSRC = kGradF16>
+template <typename T, bool DQ, bool DK, int GSRC>
 int launch_bcast_bwd_t(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
-                       const BcPlan& p, hipStream_t st, KernGrad kg) {
-  if constexpr (std::is_same<T, f16s>::value) {
-    switch (d.M) {
-      case 16: return launch_bcast_bwd_mc<T, 16, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
-      case 32: return launch_bcast_bwd_mc<T, 32, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
-      default: return launch_bcast_bwd_mc<T, 49, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
-    }
-  } else {
-    if (d.M == 16) return launch_bcast_bwd_mc<T, 16, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
-    return launch_bcast_bwd_mc<T, 49, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
-  }
+                       const BcPlan& p, hipStream_t st, const KernGrad& kg) {
+  if constexpr (std::is_same<T, f16s>::value)
+    if (d.M == 32) return launch_bcast_bwd_mc<T, 32, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
+  if (d.M == 16) return launch_bcast_bwd_mc<T, 16, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
+  return launch_bcast_bwd_mc<T, 49, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
 }
 
-// The kernel-gradient source (fp32 gK and K) is fp16-only.
 template <bool DQ, bool DK, int GSRC = kGradF16>
 int launch_bcast_bwd(int dtype, const void* g, const void* q, const void* k, void* dq, void* dk, void* ws,
-                     const Dims& d, const BcPlan& p, hipStream_t st, KernGrad kg = {}) {
-  if constexpr (GSRC == kGradF16) {
-    if (dtype == LFAMD_F32) return launch_bcast_bwd_t<float, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
-    if (dtype == LFAMD_BF16) return launch_bcast_bwd_t<bf16s, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
-  }
+                     const Dims& d, const BcPlan& p, hipStream_t st, const KernGrad& kg = {}) {
+  if (dtype == LFAMD_F32) return launch_bcast_bwd_t<float, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
+  if (dtype == LFAMD_BF16) return launch_bcast_bwd_t<bf16s, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
   return launch_bcast_bwd_t<f16s, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
 }
 
@@ -1671,14 +1828,14 @@ MbPlan plan_mb(const Dims& d, bool dkey) {
 
 template <typename T, int CB, bool DQ, bool DK, int GSRC = kGradF16>
 int launch_mb_cb(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
-                 const MbPlan& p, hipStream_t st, KernGrad kg = {}) {
+                 const MbPlan& p, hipStream_t st, const KernGrad& kg = {}) {
   auto kern = laplace_bwd_mb_kernel<T, CB, DQ, DK, GSRC>;
   if (p.lds > 65536)
     if (int s = set_dyn_lds(reinterpret_cast<const void*>(kern), p.lds, "laplace backward")) return s;
   dim3 grid(p.nx, p.ncb, (unsigned)d.BH());
   hipLaunchKernelGGL(kern, grid, dim3(64 * p.W), p.lds, st, static_cast<const T*>(g), static_cast<const T*>(q),
                      static_cast<const T*>(k), static_cast<T*>(dq), static_cast<float*>(ws), (int)d.N, (int)d.C,
-                     p.rowsPerWG, (int)d.M, kg.gk, kg.kv, kg.scale);
+                     p.rowsPerWG, (int)d.M, kg.src, kg.scale);
   int s = check_launch("laplace backward");
   if (s || !DK) return s;
   dim3 rgrid(ceil_div(64 * (int)d.M, 256), p.ncb, (unsigned)d.BH());
@@ -1689,7 +1846,7 @@ int launch_mb_cb(const void* g, const void* q, const void* k, void* dq, void* dk
 
 template <typename T, bool DQ, bool DK, int GSRC = kGradF16>
 int launch_mb_t(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
-                const MbPlan& p, hipStream_t st, KernGrad kg = {}) {
+                const MbPlan& p, hipStream_t st, const KernGrad& kg = {}) {
   switch (p.CB) {
     case 1: return launch_mb_cb<T, 1, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
     case 2: return launch_mb_cb<T, 2, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
@@ -1702,22 +1859,48 @@ int launch_mb_t(const void* g, const void* q, const void* k, void* dq, void* dk,
   }
 }
 
-template <bool DQ, bool DK>
+template <bool DQ, bool DK, int GSRC = kGradF16>
 int launch_mb(int dtype, const void* g, const void* q, const void* k, void* dq, void* dk, void* ws,
-              const Dims& d, const MbPlan& p, hipStream_t st) {
+              const Dims& d, const MbPlan& p, hipStream_t st, const KernGrad& kg = {}) {
   switch (dtype) {
-    case LFAMD_F16: return launch_mb_t<f16s, DQ, DK>(g, q, k, dq, dk, ws, d, p, st);
-    case LFAMD_BF16: return launch_mb_t<bf16s, DQ, DK>(g, q, k, dq, dk, ws, d, p, st);
-    default: return launch_mb_t<float, DQ, DK>(g, q, k, dq, dk, ws, d, p, st);
+    case LFAMD_F16: return launch_mb_t<f16s, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
+    case LFAMD_BF16: return launch_mb_t<bf16s, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
+    default: return launch_mb_t<float, DQ, DK, GSRC>(g, q, k, dq, dk, ws, d, p, st, kg);
   }
 }
 
-// The fused kernel-gradient backward (fp16): M in {16, 32, 49} on the
+// lfamd_laplace_kernel_backward_rows replaced, for bf16 / fp32 layers (M <= 64), three
+// times {g = -s gK K as an elementwise pass, casts, backward, reduction} by one launch:
+// B=2 H=2 14x14 d=32 fp32 layer step 198 -> 136 us, B=64 H=4 14x14 d=32 bf16 259 -> 148 us
+// (the three backwards 24 us each with half their lanes idle at d = 32).
+// The fused kernel-gradient backward: M in {16, 49} (fp16: 32 too) on the
 // register-resident-column kernel, any other 17 <= M <= 256 on the column-block
 // kernel (the former spills at M = 64: 94 us there against 87 us composed).
-bool kernel_bwd_bcast(const Dims& d) { return d.M == 16 || d.M == 32 || d.M == 49; }
-bool kernel_bwd_ok(int dtype, const Dims& d) {
-  return dtype == LFAMD_F16 && (kernel_bwd_bcast(d) || (d.M >= 17 && d.M <= 8 * kMbMC));
+bool kernel_bwd_bcast(int dtype, const Dims& d) { return d.M == 16 || d.M == 49 || (d.M == 32 && dtype == LFAMD_F16); }
+bool kernel_bwd_shape(int dtype, const Dims& d) {
+  return kernel_bwd_bcast(dtype, d) || (d.M >= 17 && d.M <= 8 * kMbMC);
+}
+bool kernel_bwd_ok(int dtype, const Dims& d) { return dtype == LFAMD_F16 && kernel_bwd_shape(dtype, d); }
+
+// The row sets of a kernel-gradient backward; `unit` is what the sets' ends count
+// (rows, or the column-block kernel's row batches). d.N is their total.
+KernGrad kern_grad(int nsrc, const float* const* gk, const float* const* kv, const void* const* q, void* const* dq,
+                   const int64_t* lens, int unit, float scale) {
+  KernGrad kg;
+  int end = 0;
+  for (int i = 0; i < 3; ++i) {
+    if (i < nsrc) {
+      kg.src.gk[i] = gk[i];
+      kg.src.kv[i] = kv[i];
+      kg.src.q[i] = q[i];
+      kg.src.dq[i] = dq[i];
+      kg.src.len[i] = (int)lens[i];
+      end += ceil_div((int)lens[i], unit);
+    }
+    kg.src.end[i] = end;
+  }
+  kg.scale = scale;
+  return kg;
 }
 
 template <typename T, int JB, bool DQ, bool DK>
@@ -2029,27 +2212,90 @@ int lfamd_laplace_kernel_backward(int dtype, const float* grad_kernel, const flo
   if (b2_ok(dtype, d.BH(), d.N, d.M, d.C) && (reinterpret_cast<uintptr_t>(query) & 3) == 0)
     return b2_launch(dtype, nullptr, query, key, grad_query, grad_key, workspace, workspace_bytes, d.BH(), d.N, d.M,
                      d.C, st, who, B2Grad{grad_kernel, kernel, scale});
-  const KernGrad kg{grad_kernel, kernel, scale};
-  if (!kernel_bwd_bcast(d)) {
+  const bool bcast = kernel_bwd_bcast(dtype, d);
+  const KernGrad kg = kern_grad(1, &grad_kernel, &kernel, &query, &grad_query, &q_len, bcast ? 1 : kMbRB, scale);
+  if (!bcast) {
     const MbPlan mp = plan_mb(d, doDk);
     if (doDk && (!workspace || workspace_bytes < mp.partialElems * 4))
       return fail(LFAMD_ERR_ARG, "%s: workspace of %zu bytes needed, %zu given", who, mp.partialElems * 4,
                   workspace_bytes);
     if (doDq && doDk)
-      return launch_mb_t<f16s, true, true, kGradKernel>(nullptr, query, key, grad_query, grad_key, workspace, d, mp, st, kg);
+      return launch_mb<true, true, kGradKernel>(dtype, nullptr, query, key, grad_query, grad_key, workspace, d, mp, st, kg);
     if (doDq)
-      return launch_mb_t<f16s, true, false, kGradKernel>(nullptr, query, key, grad_query, nullptr, workspace, d, mp, st, kg);
-    return launch_mb_t<f16s, false, true, kGradKernel>(nullptr, query, key, nullptr, grad_key, workspace, d, mp, st, kg);
+      return launch_mb<true, false, kGradKernel>(dtype, nullptr, query, key, grad_query, nullptr, workspace, d, mp, st, kg);
+    return launch_mb<false, true, kGradKernel>(dtype, nullptr, query, key, nullptr, grad_key, workspace, d, mp, st, kg);
   }
   const BcPlan sp = plan_bcast(d, doDk);
   if (doDk && (!workspace || workspace_bytes < sp.partialElems * 4))
     return fail(LFAMD_ERR_ARG, "%s: workspace of %zu bytes needed, %zu given", who, sp.partialElems * 4,
                 workspace_bytes);
   if (doDq && doDk)
-    return launch_bcast_bwd<true, true, kGradKernel>(LFAMD_F16, nullptr, query, key, grad_query, grad_key, workspace, d, sp, st, kg);
+    return launch_bcast_bwd<true, true, kGradKernel>(dtype, nullptr, query, key, grad_query, grad_key, workspace, d, sp, st, kg);
   if (doDq)
-    return launch_bcast_bwd<true, false, kGradKernel>(LFAMD_F16, nullptr, query, key, grad_query, nullptr, workspace, d, sp, st, kg);
-  return launch_bcast_bwd<false, true, kGradKernel>(LFAMD_F16, nullptr, query, key, nullptr, grad_key, workspace, d, sp, st, kg);
+    return launch_bcast_bwd<true, false, kGradKernel>(dtype, nullptr, query, key, grad_query, nullptr, workspace, d, sp, st, kg);
+  return launch_bcast_bwd<false, true, kGradKernel>(dtype, nullptr, query, key, nullptr, grad_key, workspace, d, sp, st, kg);
+}
+
+namespace {
+// The row sets' total as one row count: the plans' rows, padded to whole row batches per
+// set where the column-block kernel takes them.
+int rows_bwd_dims(int dtype, int nsrc, const int64_t* lens, Dims& d, const char* who) {
+  if (nsrc < 1 || nsrc > 3 || !lens) return fail(LFAMD_ERR_ARG, "%s: 1 to 3 sources expected", who);
+  int64_t rows = 0;
+  for (int i = 0; i < nsrc; ++i) {
+    if (lens[i] < 1) return fail(LFAMD_ERR_ARG, "%s: source %d has no rows", who, i);
+    if (lens[i] > INT32_MAX / 8)
+      return fail(LFAMD_ERR_UNSUPPORTED, "%s: source %d has %lld rows (at most %d)", who, i, (long long)lens[i],
+                  INT32_MAX / 8);
+    rows += kernel_bwd_bcast(dtype, d) ? lens[i] : round_up((int)lens[i], kMbRB);
+  }
+  d.N = rows;
+  if (dtype == LFAMD_F64 || !kernel_bwd_shape(dtype, d) || d.C < 1 || d.BH() < 1 || d.BH() > 65535 ||
+      ceil_div((int)d.C, 64) > 65535)
+    return fail(LFAMD_ERR_UNSUPPORTED, "%s: no fused path for dtype %d, M=%lld, C=%lld", who, dtype, (long long)d.M,
+                (long long)d.C);
+  return LFAMD_OK;
+}
+}  // namespace
+
+size_t lfamd_laplace_kernel_backward_rows_workspace_size(int dtype, int num_sources, const int64_t* q_lens,
+                                                         int64_t batch, int64_t heads, int64_t k_len,
+                                                         int64_t channels) {
+  const char* who = "laplace kernel backward (row sets)";
+  Dims d{batch, heads, 1, k_len, channels};
+  if (!valid_dtype(dtype) || check_dims(d, who) || rows_bwd_dims(dtype, num_sources, q_lens, d, who)) return 0;
+  return (kernel_bwd_bcast(dtype, d) ? plan_bcast(d, true).partialElems : plan_mb(d, true).partialElems) * 4;
+}
+
+int lfamd_laplace_kernel_backward_rows(int dtype, int num_sources, const float* const* grad_kernels,
+                                       const float* const* kernels, const void* const* queries,
+                                       const int64_t* q_lens, const void* key, void* const* grad_queries,
+                                       void* grad_key, int64_t batch, int64_t heads, int64_t k_len,
+                                       int64_t channels, float scale, void* workspace, size_t workspace_bytes,
+                                       void* stream) {
+  const char* who = "laplace kernel backward (row sets)";
+  if (!valid_dtype(dtype)) return fail(LFAMD_ERR_DTYPE, "%s: unsupported dtype %d", who, dtype);
+  Dims d{batch, heads, 1, k_len, channels};
+  int s = check_dims(d, who);
+  if (s || (s = rows_bwd_dims(dtype, num_sources, q_lens, d, who))) return s;
+  if (!grad_kernels || !kernels || !queries || !grad_queries || !key || !grad_key)
+    return fail(LFAMD_ERR_ARG, "%s: null pointer", who);
+  for (int i = 0; i < num_sources; ++i)
+    if (!grad_kernels[i] || !kernels[i] || !queries[i] || !grad_queries[i])
+      return fail(LFAMD_ERR_ARG, "%s: null pointer", who);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool bcast = kernel_bwd_bcast(dtype, d);
+  const KernGrad kg = kern_grad(num_sources, grad_kernels, kernels, queries, grad_queries, q_lens,
+                                bcast ? 1 : kMbRB, scale);
+  const BcPlan bp = bcast ? plan_bcast(d, true) : BcPlan{};
+  const MbPlan mp = bcast ? MbPlan{} : plan_mb(d, true);
+  const size_t need = (bcast ? bp.partialElems : mp.partialElems) * 4;
+  if (!workspace || workspace_bytes < need)
+    return fail(LFAMD_ERR_ARG, "%s: workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
+  return bcast ? launch_bcast_bwd<true, true, kGradKernel>(dtype, nullptr, nullptr, key, nullptr, grad_key, workspace,
+                                                           d, bp, st, kg)
+               : launch_mb<true, true, kGradKernel>(dtype, nullptr, nullptr, key, nullptr, grad_key, workspace, d, mp,
+                                                    st, kg);
 }
 
 int lfamd_laplace_reduce_forward(int dtype, const void* query, const void* key,

@@ -6,6 +6,8 @@
 // src/NewtonInverse_cuda_kernel.cu:17-19).
 #pragma once
 
+#include <type_traits>
+#include <utility>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -120,5 +122,14 @@ __device__ __forceinline__ float half_step(float d) {
 
 __host__ __device__ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 __host__ __device__ constexpr int round_up(int a, int b) { return ceil_div(a, b) * b; }
+
+// f(0), ..., f(N - 1) with compile-time arguments.
+template <typename F, int... I>
+__device__ __forceinline__ void unrolled_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F> __device__ __forceinline__ void unrolled(F&& f) {
+  unrolled_impl(f, std::make_integer_sequence<int, N>{});
+}
 
 }  // namespace lfamd

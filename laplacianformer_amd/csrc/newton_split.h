@@ -654,15 +654,6 @@ struct SplitTask {
   }
 };
 
-// f(0), ..., f(N - 1) with compile-time arguments.
-template <typename F, int... I>
-__device__ __forceinline__ void unrolled_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F> __device__ __forceinline__ void unrolled(F&& f) {
-  unrolled_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 template <int NR, int KS> struct WideLayout {
   static constexpr int NP = 32 * NR;
   static constexpr int LS = NP + 4;

@@ -159,6 +159,33 @@ bool LaplaceKernel_backward_cuda(const at::Tensor gradKernel, const at::Tensor k
       (float)scale, ws.data_ptr(), ws_bytes, detail::stream_of(query)));
 }
 
+bool LaplaceKernel_backward_rows(const at::Tensor gradKernel, const at::Tensor kernel, const at::Tensor query,
+                                 const at::Tensor key, at::Tensor gradQuery, at::Tensor gradKey, double scale) {
+  TORCH_CHECK(gradKernel.is_cuda() && query.is_cuda() && key.is_cuda(), "laplace kernel backward: GPU tensors expected");
+  shape_check(query, key);
+  const int dt = detail::abi_dtype(query, "laplace_kernel_backward");
+  detail::same_type(query, key, "key");
+  const Sizes s = sizes_of(query, key);
+  check_kernel_tensor(query, kernel, s, "kernel");
+  TORCH_CHECK(gradKernel.scalar_type() == at::kFloat && gradKernel.sizes() == kernel.sizes(),
+              "gradKernel must be float32 of the kernel's shape");
+  check_out(query, gradQuery, {s.B, s.H, s.N, s.C}, "gradQuery");
+  check_out(query, gradKey, {s.B, s.H, s.C, s.M}, "gradKey");
+  at::hip::HIPGuardMasqueradingAsCUDA guard(query.device());
+  const int64_t n = s.N;
+  const size_t wsb = lfamd_laplace_kernel_backward_rows_workspace_size(dt, 1, &n, s.B, s.H, s.M, s.C);
+  if (wsb == 0) return false;
+  const at::Tensor gk = gradKernel.contiguous();
+  at::Tensor ws = at::empty({(int64_t)wsb}, query.options().dtype(at::kByte));
+  const float* gkp = gk.data_ptr<float>();
+  const float* kvp = kernel.data_ptr<float>();
+  const void* qp = query.data_ptr();
+  void* dqp = gradQuery.data_ptr();
+  return fused_status(lfamd_laplace_kernel_backward_rows(dt, 1, &gkp, &kvp, &qp, &n, key.data_ptr(), &dqp,
+                                                         gradKey.data_ptr(), s.B, s.H, s.M, s.C, (float)scale,
+                                                         ws.data_ptr(), wsb, detail::stream_of(query)));
+}
+
 void LaplaceSubtraction_reduce_forward_cuda(const at::Tensor query, const at::Tensor key, at::Tensor output) {
   shape_check(query, key);
   const int dt = detail::abi_dtype(query, "subtraction_reduce_laplace_forward_cuda");

@@ -242,6 +242,16 @@ std::vector<at::Tensor> LaplacianAttention_backward(at::Tensor g, std::vector<at
                                                km_cm.size(3), dd, (float)s, ws.data_ptr(), wsb,
                                                detail::stream_of(k));
     }
+    if (st == LFAMD_ERR_UNSUPPORTED && d_kqm.is_contiguous() && d_kkm.is_contiguous() && d_kmm.is_contiguous()) {
+      const size_t rwsb =
+          lfamd_laplace_kernel_backward_rows_workspace_size(dt, 3, ns, B, H, km_cm.size(3), dd);
+      if (rwsb > 0) {
+        at::Tensor ws = at::empty({(int64_t)rwsb}, k.options().dtype(at::kByte));
+        st = lfamd_laplace_kernel_backward_rows(dt, 3, gks, kvs, qs, ns, km_cm.data_ptr(), dqs, d_cm.data_ptr(), B, H,
+                                                km_cm.size(3), dd, (float)s, ws.data_ptr(), rwsb,
+                                                detail::stream_of(k));
+      }
+    }
     if (st == LFAMD_ERR_UNSUPPORTED) {
       std::tie(d_q, d_cm) = kernel_bwd(d_kqm, k_qm, q, km_cm, s);
       std::tie(d_km, d_cm2) = kernel_bwd(d_kmm, k_mm, km, km_cm, s);

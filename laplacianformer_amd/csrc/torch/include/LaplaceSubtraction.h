@@ -30,6 +30,10 @@ bool LaplaceKernel_forward_cuda(const at::Tensor query, const at::Tensor key, at
 bool LaplaceKernel_backward_cuda(const at::Tensor gradKernel, const at::Tensor kernel, const at::Tensor query,
                                  const at::Tensor key, std::optional<at::Tensor> gradQuery,
                                  std::optional<at::Tensor> gradKey, double scale);
+// Both gradients for any of the three types (lfamd_laplace_kernel_backward_rows with one
+// row set); false where that path does not apply.
+bool LaplaceKernel_backward_rows(const at::Tensor gradKernel, const at::Tensor kernel, const at::Tensor query,
+                                 const at::Tensor key, at::Tensor gradQuery, at::Tensor gradKey, double scale);
 // LaplacianFormer attention layer's row products (no reference counterpart):
 // C[..., n, q] = sum_p A[..., n, p] * B[..., q, p] for a small B read through its
 // strides, inner and output widths <= 64 (lfamd_mix_rows).

@@ -60,6 +60,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("LaplaceKernel_backward", &LaplaceKernel_backward,
         "LaplaceKernel_backward (gradKernel, kernel, query, key, gradQuery, gradKey, scale): "
         "gradQuery / gradKey may be None; False where the fused path does not apply");
+#if defined(WITH_HIP)
+  m.def("LaplaceKernel_backward_rows", &LaplaceKernel_backward_rows,
+        "LaplaceKernel_backward_rows (gradKernel, kernel, query, key, gradQuery, gradKey, scale): both gradients, "
+        "fp16 / bf16 / fp32; False where the fused path does not apply");
+#endif
   m.def("MixRows", &MixRows,
         "MixRows (a, b, c): c[..., n, q] = sum_p a[..., n, p] * b[..., q, p] in float32, widths <= 64 "
         "(the attention layer's products; b is read through its strides)");

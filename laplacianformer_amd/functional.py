@@ -88,6 +88,9 @@ class LaplaceKernelFunction(torch.autograd.Function):
         dk = torch.empty_like(key) if need_k else None
         if kern.dtype == torch.float32 and ext().LaplaceKernel_backward(grad, kern, query, key, dq, dk, ctx.scale):
             return dq, dk, None
+        if kern.dtype == torch.float32 and need_q and need_k \
+                and ext().LaplaceKernel_backward_rows(grad, kern, query, key, dq, dk, ctx.scale):
+            return dq, dk, None
         acc = kern.dtype
         g = grad * kern * -ctx.scale
         qa, ka = query.to(acc), key.to(acc)

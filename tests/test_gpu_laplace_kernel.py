@@ -289,3 +289,95 @@ def test_kernel_forward_multi_rejects(gpu):
     assert f(1, 0, 49) == 1 and f(1, 4, 49) == 1   # 1 to 3 sources
     assert f(1, 1, 48) == 3                        # M != 49 (LFAMD_ERR_UNSUPPORTED)
     assert f(3, 1, 49) == 3                        # fp64
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("lens,bh,M,C", [((49, 196, 196), (2, 4), 49, 32), ((7, 1, 30), (1, 3), 49, 20),
+                                         ((196, 196, 49), (32, 8), 49, 32), ((33, 130), (1, 2), 49, 96),
+                                         ((16, 65, 9), (1, 2), 16, 31), ((64, 129, 3), (1, 2), 32, 64),
+                                         ((50, 71, 8), (1, 2), 50, 40), ((196, 333, 1), (1, 2), 196, 64),
+                                         ((17,), (1, 1), 255, 65)],
+                         ids=lambda s: "-".join(map(str, s)) if isinstance(s, tuple) else str(s))
+def test_kernel_backward_rows(gpu, dt, lens, bh, M, C):
+    """lfamd_laplace_kernel_backward_rows: up to three row sets against one key in one launch, every
+    type, on the register-column kernel (M = 16, 49; two rows per wave at C <= 32, the last one
+    without a partner; one workgroup per slice stores grad_key itself, more go through the partial
+    sums) and the column-block kernel (other M, a partial last block, row batches ending with their
+    set). grad_query and the summed grad_key against the oracle in fp64, the usual bounds."""
+    import ctypes
+
+    import laplacianformer_amd as lf
+
+    B, H = bh
+    print(f"laplace kernel backward rows {dt} {lens} B={B} H={H} M={M} C={C}", flush=True)
+    lib = lf.capi()
+    s = 1.0 / math.sqrt(C)
+    k = gen((B, H, C, M), 871, dt)
+    srcs = []
+    for i, n in enumerate(lens):
+        q = gen((B, H, n, C), 872 + i, dt)
+        gk = gen((B, H, n, M), 882 + i, "f32")
+        kern = torch.exp(-torch.rand((B, H, n, M), generator=torch.Generator().manual_seed(892 + i)) * 4)
+        srcs.append((q, gk, kern))
+    kd = k.to(gpu)
+    qd, gkd, kvd = ([src[i].to(gpu) for src in srcs] for i in range(3))
+    dqs, dk = [torch.empty_like(q) for q in qd], torch.empty_like(kd)
+    ns = len(lens)
+    nl = (ctypes.c_int64 * ns)(*lens)
+    P = lambda ts: (ctypes.c_void_p * ns)(*[t.data_ptr() for t in ts])  # noqa: E731
+    code = lf.dtype_code(kd)
+    wsb = lib.lfamd_laplace_kernel_backward_rows_workspace_size(code, ns, nl, B, H, M, C)
+    assert wsb > 0
+    ws = torch.empty(wsb, dtype=torch.uint8, device=gpu)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    call = lambda n: lib.lfamd_laplace_kernel_backward_rows(  # noqa: E731
+        code, ns, P(gkd), P(kvd), P(qd), nl, kd.data_ptr(), P(dqs), dk.data_ptr(), B, H, M, C, ctypes.c_float(s),
+        ws.data_ptr(), n, stream)
+    assert call(wsb - 1) == 1  # workspace too small: refused before any launch
+    lf.check(call(wsb))
+    rk, scale = 0.0, 0.0
+    for (q, gk, kern), dq in zip(srcs, dqs):
+        g64 = -s * gk.double().numpy() * kern.double().numpy()
+        ga = np.abs(g64)
+        rq = oracle.laplace_backward_query(g64, q, k, "f64")
+        assert_l1_close(dq, rq, dt, "dq", np.broadcast_to(ga.sum(axis=3, keepdims=True), rq.shape))
+        rk = rk + oracle.laplace_backward_key(g64, q, k, "f64")
+        scale = scale + ga.sum(axis=2, keepdims=True)
+    assert_l1_close(dk, rk, dt, "dk (sum over the sets)", np.broadcast_to(scale, rk.shape))
+
+
+@pytest.mark.parametrize("M,C", [(49, 64), (16, 20), (196, 64)])
+@pytest.mark.parametrize("keys", ["subnormal", "huge", "inf"])
+def test_f32_step_range(gpu, M, C, keys):
+    """The fp32 backward's step at the ends of the type's range: differences of one subnormal unit,
+    queries that overflow when scaled, and keys at, above and far above the bound of the scaled
+    step (the unscaled one takes those): exact signs, so the usual bounds."""
+    import laplacianformer_amd as lf
+
+    B, H, N = 1, 2, 37
+    print(f"f32 step range M={M} C={C} keys={keys}", flush=True)
+    q, k, g = gen((B, H, N, C), 911, "f32"), gen((B, H, C, M), 912, "f32"), gen((B, H, N, M), 913, "f32")
+    tiny = torch.tensor(2.0 ** -149)
+    q[..., ::2, :] = torch.round(q[..., ::2, :] * 2) * tiny   # ties and one-unit differences
+    q[:, :, 1] *= 2.0 ** 125                                   # overflow once scaled
+    k[..., ::3] = torch.round(k[..., ::3] * 2) * tiny
+    if keys == "huge":
+        k[0, 0, 0, :3] = torch.tensor([2.0 ** 103, -3.0e38, 3.0e38])
+        q[0, 0, 0, 0] = 2.0 ** 103
+    if keys == "inf":
+        k[0, 1, 1, :2] = torch.tensor([float("inf"), float("-inf")])
+    qd, kd, gd = q.to(gpu), k.to(gpu), g.to(gpu)
+    dq, dk = torch.empty_like(qd), torch.empty_like(kd)
+    sg = torch.sign(q.double()[..., None] - k.double()[:, :, None])  # [B,H,N,C,M]
+    rq = (g.double()[:, :, :, None] * sg).sum(-1).numpy()
+    rk = -(g.double()[:, :, :, None] * sg).sum(2).numpy()
+    ga = g.double().abs()
+    L = lf.ext()
+    for both in (False, True):
+        if both:
+            L.LaplaceSubtraction_backward(gd, qd, kd, dq, dk)
+        else:
+            L.LaplaceSubtraction_backward_query(gd, qd, kd, dq)
+            L.LaplaceSubtraction_backward_key(gd, qd, kd, dk)
+        assert_l1_close(dq, rq, "f32", "dq", np.broadcast_to(ga.sum(3, keepdim=True).numpy(), rq.shape))
+        assert_l1_close(dk, rk, "f32", "dk", np.broadcast_to(ga.sum(2, keepdim=True).numpy(), rk.shape))
