@@ -690,14 +690,15 @@ __device__ __forceinline__ void store_tiles(float* __restrict__ dst, int wave, i
 }
 
 // The landmark forward in two launches. First, workgroups [0, bh) run
-// NewtonInverse on the bh landmark matrices (the bodies that lfamd_newton_forward
-// runs below two matrices per CU, writing the inverse) and workgroups [bh, bh (1 + per)) the tall product's partials of
-// K_km^T V (tall_t_bf16_body, per workgroups per slice): the two sets share
-// nothing, so the memory-bound tall product runs on the CUs that the
-// latency-bound iterations leave free. Then landmark_kv_w_kernel sums the
-// partials into kv (in workgroup order) and forms W = inv kv. One block size
-// serves both roles: 512 threads, two waves per 16-row strip of NewtonInverse
-// (the tall body needs more registers than 1024-thread blocks allow).
+// NewtonInverse on the bh landmark matrices (the body that lfamd_newton_forward
+// takes for them: the symmetric one for m = 49, else the chain body, so this kernel
+// runs only where that entry takes the chain kernel) and workgroups [bh, bh (1 + per))
+// the tall product's partials of K_km^T V (tall_t_bf16_body, per workgroups per
+// slice): the two sets share nothing, so the memory-bound tall product runs on the
+// CUs that the latency-bound iterations leave free. Then landmark_kv_w_kernel sums
+// the partials into kv (in workgroup order) and forms W = inv kv. One block size
+// serves both roles: 512 threads (the tall body needs more registers than 1024-thread
+// blocks allow), of which the chain body takes the first four waves.
 template <int NP, int KL, typename TB>
 __global__ void __launch_bounds__(NP * 8)
 newton_fwd_tall_kernel(const float* __restrict__ kmm, float* __restrict__ inv, int n, int iters, int bh,
@@ -1434,9 +1435,11 @@ int launch_fwd(Kern k, int64_t blocks, int threads, size_t lds, hipStream_t st, 
 // products leave the SIMD to the splitting (1024 x 64^2, 12 iterations: 70.0 against
 // 59.5 us, 512: 42 against 29.5; below, a matrix's latency counts: 32 matrices 18.9 us).
 // n > 64: one workgroup of 32-column waves per matrix and CU.
+bool fwd_many(int64_t bh) { return bh >= 2 * (int64_t)num_cus(); }
+
 template <typename T, int NP>
 int fwd_np(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
-  const bool many = bh >= 2 * (int64_t)num_cus();
+  const bool many = fwd_many(bh);
   // fp32 n = 49: the symmetric iteration when P is symmetric (the kernel checks; else the general one).
   if constexpr (std::is_same<T, float>::value && NP == 64)
     if (n == 49)
@@ -1663,6 +1666,15 @@ int lfamd_attention_landmarks_forward(const float* kmm, const float* kkm, int v_
   float* part = static_cast<float*>(workspace);
   if (iters < 0) iters = 0;
   if (int s = tall_t_check(v_dtype, kkm, v, workspace_bytes, slices, rows, m, d, &per)) return s;
+  if (m != 49 && fwd_many(slices)) {
+    // Two matrices per CU and more: lfamd_newton_forward's kernel for them, which no CU has
+    // room beside, then the tall product (196 rows, m = 64, 10 iterations: 512 slices 62.2
+    // against 70.4 us with the chain body beside the tall product, 1024 102.8 against 127.5,
+    // 600, the last of three rounds nearly empty, 84 either way).
+    if (int s = fwd_np<float, 64>(kmm, inv, slices, m, iters, st)) return s;
+    if (int s = tall_t_partials(v_dtype, kkm, v, part, workspace_bytes, slices, rows, m, d, st, &per)) return s;
+    return launch_kv_w<4>(inv, part, per, slices, m, d, kv, w, st);
+  }
   if (int s = (m == 49 ? launch_fwd_tall<1>(v_dtype, kmm, inv, slices, m, iters, kkm, v, part, rows, d, per, st)
                        : launch_fwd_tall<4>(v_dtype, kmm, inv, slices, m, iters, kkm, v, part, rows, d, per, st)))
     return s;

@@ -35,7 +35,10 @@ def _close(got, ref, scale, what):
     (3, 784, 49, 64, "f16"),      # the layer's shape: one live row in the last strip (KL = 1)
     (5, 200, 64, 64, "f32"),      # a full 64 bucket
     (4, 96, 56, 16, "bf16"),      # a partial bucket, narrow d
-    (600, 32, 49, 32, "f16"),     # more than two matrices per CU: two waves per strip
+    (600, 32, 49, 32, "f16"),     # more than two matrices per CU
+    (511, 40, 64, 64, "f16"),     # the last count of the fused launch, m != 49
+    (512, 33, 64, 64, "f32"),     # from here on lfamd_newton_forward's two-wave kernel
+    (601, 32, 56, 16, "bf16"),
 ])
 def test_landmarks_forward(gpu, slices, rows, m, d, vdt):
     import laplacianformer_amd as lf
