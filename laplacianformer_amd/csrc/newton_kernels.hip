@@ -1575,7 +1575,9 @@ constexpr size_t kMulBwdLds = 4 * (size_t)NsLayout<64>::ELEMS * 4;
 template <int KL>
 int launch_fwd_tall(int v_dtype, const float* kmm, float* inv, int64_t bh, int m, int iters, const float* kkm,
                     const void* v, float* part, int64_t rows, int d, int per, hipStream_t st) {
-  const size_t lds = std::max<size_t>(fwd_lds<64>(), (size_t)tall_lds_floats() * 4);
+  // The roles' needs: the symmetric body or the chain body, and the tall product's tiles.
+  constexpr size_t inverse = KL == 1 ? fwd_lds<64>() : (size_t)ChainLayout<4>::LDS;
+  const size_t lds = std::max(inverse, (size_t)tall_lds_floats() * 4);
   const dim3 grid((unsigned)(bh * (1 + per))), block(64 * 8);
   auto go = [&](auto k, const auto* B) -> int {
     if (int s = check_fit(reinterpret_cast<const void*>(k), 64 * 8, lds, "attention landmarks forward")) return s;
