@@ -268,8 +268,8 @@ template <int NP, int WPR, int KL> constexpr bool fwd_va() { return KL == 1 && W
 
 // V <- 2V - V(PV) (the reference's order for n <= 112) on the fp32 matrix cores, P
 // held in registers as this wave's A operand after the set-up, so the LDS holds V
-// and T = PV only. For n <= 16, and fp32 n = 49 where P is not symmetric; the other
-// sizes run on the kernels of newton_split.h.
+// and T = PV only. For n <= 16, fp32 n = 49 where P is not symmetric, and where
+// fwd_on_fp32 below says so; else the kernels of newton_split.h.
 template <typename T, int NP, int WPR, int KL>
 __device__ __forceinline__ void newton_fwd_body(const T* __restrict__ mat, T* __restrict__ out, int n, int iters) {
   using L = NsLayout<NP, WPR>;
@@ -635,10 +635,10 @@ newton_fwd_sym_kernel(const float* __restrict__ mat, float* __restrict__ out, in
   newton_fwd_sym_body<NW>(mat, out, n, iters);
 }
 
-template <typename T, int NP>
-__global__ void __launch_bounds__(NP * 4)
+template <typename T, int NP, int WPR, int KL>
+__global__ void __launch_bounds__(NP * 4 * WPR)
 newton_fwd_kernel(const T* __restrict__ mat, T* __restrict__ out, int n, int iters) {
-  newton_fwd_body<T, NP, 1, 4>(mat, out, n, iters);
+  newton_fwd_body<T, NP, WPR, KL>(mat, out, n, iters);
 }
 
 // ---------------------------------------------------------------------------
@@ -1437,6 +1437,42 @@ int launch_fwd(Kern k, int64_t blocks, int threads, size_t lds, hipStream_t st, 
 // n > 64: one workgroup of 32-column waves per matrix and CU.
 bool fwd_many(int64_t bh) { return bh >= 2 * (int64_t)num_cus(); }
 
+template <int NP> constexpr int narrow_wpr() { return pick_wpr<NP>() == 4 ? 2 : pick_wpr<NP>(); }
+
+// Where the products stay on the fp32 matrix instructions: no iteration (V0 = alpha P as
+// it is), or too few for the pieces' set-up and their one workgroup per matrix:
+//   n <= 32    up to two matrices per CU, whose two waves have nothing to hide the splitting
+//              behind (512 x 32^2, 12 iterations 12.1 against 14.9 us, 8 matrices 9.7 / 10.5;
+//              600 15.6 / 15.0, 1024 18.7 / 16.4), and two iterations (1024, one: 5.5 / 5.7);
+//   49 .. 64   one iteration (bf16 512 x 64^2 9.8 against 12.4 us), two below two matrices
+//              per CU (8 matrices 7.9 / 8.4; 512 x 64^2 14.4 / 11.6);
+//   65 .. 96   two iterations above one matrix per CU, where several of this kernel share one
+//              (512 x 80^2: one 22.6 against 27.1 us, two 32.8 / 35.0, three 42.7 / 41.6);
+//   113 .. 128 two iterations, three above 64 matrices, four from one per CU on: the wide
+//              kernel's spilled third pieces cost 20 to 50 us a call (256 x 128^2: one 26.7 against
+//              67.4 us, four 73.6 / 94.2, six about 106 / 114; 128 matrices, three, 57 / 71).
+// fp32 n = 17 and 65 always: row 16 (64) runs on the VALU beside the strips, where the pieces
+// pad it to a tile (1024 x 17^2, 12 iterations 11.5 against 15.7 us; 512 x 65^2 82.5 / 111).
+template <int NP> bool fwd_on_fp32(int64_t bh, int iters) {
+  const bool many = fwd_many(bh);
+  if (iters == 0) return true;
+  if (NP == 32) return iters <= 2 || bh <= 2 * (int64_t)num_cus();
+  if (NP == 64) return iters <= (many ? 1 : 2);
+  if (NP == 80 || NP == 96) return iters <= 2 && bh > num_cus();
+  if (NP == 128) return iters <= (bh >= num_cus() ? 4 : bh > num_cus() / 4 ? 3 : 2);
+  return false;
+}
+
+// The most waves per strip while there are fewer than two matrices per CU (latency-bound);
+// with more, two per strip at most keep more matrices resident.
+template <typename T, int NP, int KL>
+int fwd_fp32(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
+  constexpr int W = pick_wpr<NP>(), V = narrow_wpr<NP>();
+  if (V != W && fwd_many(bh))
+    return launch_fwd(newton_fwd_kernel<T, NP, V, KL>, bh, NP * 4 * V, fwd_lds<NP>(), st, m, o, n, iters);
+  return launch_fwd(newton_fwd_kernel<T, NP, W, KL>, bh, NP * 4 * W, fwd_lds<NP>(), st, m, o, n, iters);
+}
+
 template <typename T, int NP>
 int fwd_np(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
   const bool many = fwd_many(bh);
@@ -1445,8 +1481,11 @@ int fwd_np(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
     if (n == 49)
       return many ? launch_fwd(newton_fwd_sym_kernel<8>, bh, 512, fwd_lds<NP>(), st, m, o, n, iters)
                   : launch_fwd(newton_fwd_sym_kernel<16>, bh, 1024, fwd_lds<NP>(), st, m, o, n, iters);
+  if constexpr (std::is_same<T, float>::value && (NP == 32 || NP == 80))
+    if (n == NP - 15) return fwd_fp32<T, NP, 1>(m, o, bh, n, iters, st);
+  if (NP == 16 || fwd_on_fp32<NP>(bh, iters)) return fwd_fp32<T, NP, 4>(m, o, bh, n, iters, st);
   if constexpr (NP == 16) {
-    return launch_fwd(newton_fwd_kernel<T, NP>, bh, NP * 4, fwd_lds<NP>(), st, m, o, n, iters);
+    return LFAMD_OK;  // (not reached: the pieces' kernels have no 16 bucket)
   } else if constexpr (NP <= 64) {
     constexpr int NT = NP / 16;
     if constexpr (NP == 64)
@@ -1454,7 +1493,7 @@ int fwd_np(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
         return launch_fwd(newton_fwd_tile_kernel<T>, (bh + 1) / 2, 256, 2 * TileLayout::LDS, st, m, o, bh, n, iters);
     return launch_fwd(newton_fwd_chain_kernel<T, NT>, bh, 64 * NT, ChainLayout<NT>::LDS, st, m, o, n, iters);
   } else {
-    constexpr int NR = (NP + 31) / 32, KS = std::is_same<T, float>::value ? NP / 16 : 2 * NR;
+    constexpr int NR = (NP + 31) / 32, KS = NP / 16;
     return launch_fwd(newton_fwd_wide_kernel<T, NR, KS>, bh, 64 * NR, WideLayout<NR, KS>::LDS, st, m, o, n, iters);
   }
 }
@@ -1493,8 +1532,6 @@ int bwd_np_w(const T* g, const T* v, T* o, int64_t bh, int n, hipStream_t st) {
   hipLaunchKernelGGL(k, dim3((unsigned)bh), dim3(NP * 4 * WPR), lds, st, g, v, o, n);
   return check_launch("newton backward");
 }
-
-template <int NP> constexpr int narrow_wpr() { return pick_wpr<NP>() == 4 ? 2 : pick_wpr<NP>(); }
 
 // The backward's two products per matrix are latency-bound at any matrix count
 // (four waves per strip: 14.5 against 15.2 us at 1024 x 64^2, where the forward's
@@ -1668,9 +1705,9 @@ int lfamd_attention_landmarks_forward(const float* kmm, const float* kkm, int v_
   float* part = static_cast<float*>(workspace);
   if (iters < 0) iters = 0;
   if (int s = tall_t_check(v_dtype, kkm, v, workspace_bytes, slices, rows, m, d, &per)) return s;
-  if (m != 49 && fwd_many(slices)) {
-    // Two matrices per CU and more: lfamd_newton_forward's kernel for them, which no CU has
-    // room beside, then the tall product (196 rows, m = 64, 10 iterations: 512 slices 62.2
+  if (m != 49 && (fwd_many(slices) || fwd_on_fp32<64>(slices, iters))) {
+    // Two matrices per CU and more, or too few iterations: lfamd_newton_forward's own kernel
+    // for them, which no CU has room beside, then the tall product (196 rows, m = 64, 10 iterations: 512 slices 62.2
     // against 70.4 us with the chain body beside the tall product, 1024 102.8 against 127.5,
     // 600, the last of three rounds nearly empty, 84 either way).
     if (int s = fwd_np<float, 64>(kmm, inv, slices, m, iters, st)) return s;

@@ -320,6 +320,27 @@ def test_newton_forward_split(gpu, bh, n, dt, iters):
     assert_newton_close(out, oracle.newton_forward(A, iters, dt), dt, f"bh={bh} n={n} {dt} it={iters}")
 
 
+@pytest.mark.parametrize("bh,n,dt,iters", [(3, 17, "f32", 9), (513, 17, "f32", 5), (513, 17, "bf16", 5),
+                                           (512, 32, "f32", 5), (513, 32, "f16", 3), (513, 30, "f32", 2),
+                                           (512, 50, "bf16", 1), (512, 50, "bf16", 2), (511, 50, "f32", 2),
+                                           (2, 65, "f32", 9), (513, 65, "f32", 3), (2, 65, "bf16", 9),
+                                           (256, 80, "f32", 2), (257, 80, "f16", 2), (257, 90, "bf16", 3),
+                                           (2, 105, "bf16", 6), (2, 105, "f16", 0), (2, 128, "f32", 2),
+                                           (65, 128, "f32", 3), (64, 128, "f16", 3), (256, 128, "f32", 4),
+                                           (256, 115, "bf16", 5)])
+def test_newton_forward_fp32_rule(gpu, bh, n, dt, iters):
+    """Both sides of the rule between the fp32 matrix instructions and the bf16 pieces (counts of
+    matrices and iterations, n = 17 and 65), on general matrices."""
+    import laplacianformer_amd as lf
+
+    print(f"newton forward rule bh={bh} n={n} {dt} iters={iters}", flush=True)
+    noise = gen((bh, n, n), 921 + n, "f64").numpy()
+    A = torch.from_numpy(gram(1, n, 64, seed=920 + n) + 1e-2 / n * noise).reshape(bh, 1, n, n).to(TORCH_DT[dt])
+    out = torch.full_like(A, float("nan"), device=gpu)
+    lf.ext().NewtonInverse_forward(A.to(gpu), out, iters)
+    assert_newton_close(out, oracle.newton_forward(A, iters, dt), dt, f"bh={bh} n={n} {dt} it={iters}")
+
+
 @pytest.mark.parametrize("bh,n", [(2, 40), (2, 64), (600, 64), (2, 100), (2, 128)])
 def test_newton_forward_split_nonfinite(gpu, bh, n):
     """A matrix with a NaN or an infinity gives no finite value after an iteration (every row
