@@ -2,9 +2,12 @@
 //
 // Every fp32 operand is held as x = p1 + p2 + p3, three bf16 pieces of 8
 // significant bits each (p1 = x rounded to bf16, p2 the rest rounded, p3 what is
-// left, exactly): no bit of x is dropped. A product takes the six piece products of
+// left): exactly for 0 and 2^-110 <= |x| < 3.39e38 (above, p1 rounds to infinity).
+// Below, p3 ends at bf16's smallest subnormal, 2^-133, which the matrix instructions
+// keep: x is held to within 2^-134. So the operands are scaled by powers of two where
+// a caller's can be out of that range. A product takes the six piece products of
 // weight 2^-16 and more (p1q1, p1q2, p2q1, p1q3, p2q2, p3q1), accumulated in fp32
-// by v_mfma_f32_16x16x32_bf16; the three left out are below 2^-24 |x| |y| each,
+// by v_mfma_f32_16x16x32_bf16; the three left out add up to less than 2^-24 |x| |y|,
 // under the rounding of one fp32 product. Six of these instructions do the work
 // of eight v_mfma_f32_16x16x4_f32 in 96 cycles instead of 256.
 #pragma once
@@ -68,6 +71,13 @@ __device__ __forceinline__ uint2 quad_transpose(uint2 d, int lane) {
   return uint2{__builtin_amdgcn_perm(nl, lo, sel), __builtin_amdgcn_perm(nh, hi, sel)};
 }
 
+// The forward kernels iterate on P / 2 and 2V, whose products are those of P and V exactly: a
+// finite P then never rounds to an infinite first piece. (Small entries need nothing: P has
+// 0.01 on its diagonal, and a finite alpha means row sums between 2^-64 and 2^64, so 2^-134 is
+// far under the rounding of P and V by norm.)
+constexpr float kHalfP = 0.5f;
+__device__ __forceinline__ float twice_v0(float alpha, float p) { return 2.0f * (alpha * p); }
+
 template <int NT> struct ChainLayout {
   static constexpr int NP = 16 * NT;
   static constexpr int KS = (NT + 1) / 2;        // 32-k steps
@@ -124,19 +134,19 @@ __device__ __forceinline__ void newton_fwd_chain_body(const T* __restrict__ Mg, 
       if (2 * u + hf < NT) v = *reinterpret_cast<const float4*>(&Ps[(16 * w + li) * LS + 32 * u + 16 * hf + 4 * lg]);
       xr[u][4 * hf] = v.x; xr[u][4 * hf + 1] = v.y; xr[u][4 * hf + 2] = v.z; xr[u][4 * hf + 3] = v.w;
     }
-  auto put_rows = [&](float s) {
+  auto put_rows = [&](auto f) {
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
       uint2 h0[3], h1[3];
-      const float a[4] = {s * xr[u][0], s * xr[u][1], s * xr[u][2], s * xr[u][3]};
-      const float b[4] = {s * xr[u][4], s * xr[u][5], s * xr[u][6], s * xr[u][7]};
+      const float a[4] = {f(xr[u][0]), f(xr[u][1]), f(xr[u][2]), f(xr[u][3])};
+      const float b[4] = {f(xr[u][4]), f(xr[u][5]), f(xr[u][6]), f(xr[u][7])};
       split_quad(a, h0);
       split_quad(b, h1);
 #pragma unroll
       for (int pc = 0; pc < 3; ++pc) op(0, w, u, pc)[lane] = uint4{h0[pc].x, h0[pc].y, h1[pc].x, h1[pc].y};
     }
   };
-  put_rows(1.0f);
+  put_rows([](float p) { return kHalfP * p; });
   // alpha = 1.8 / (max_i sum_j P_ij)^2, row sums in ascending j, one thread per row.
   float row = -1e30f;
   if ((int)threadIdx.x < n) {
@@ -169,7 +179,7 @@ __device__ __forceinline__ void newton_fwd_chain_body(const T* __restrict__ Mg, 
   for (int t = 0; t < 2 * KS; ++t) {
     if (t < NT) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vf[t][r] = alpha * Ps[(16 * t + 4 * lg + r) * LS + 16 * w + li];
+      for (int r = 0; r < 4; ++r) vf[t][r] = twice_v0(alpha, Ps[(16 * t + 4 * lg + r) * LS + 16 * w + li]);
       split_quad(vf[t], vh[t]);
     } else {
 #pragma unroll
@@ -177,7 +187,7 @@ __device__ __forceinline__ void newton_fwd_chain_body(const T* __restrict__ Mg, 
     }
   }
   __syncthreads();  // P's operands are in registers
-  put_rows(alpha);
+  put_rows([=](float p) { return twice_v0(alpha, p); });
 
   // Where this wave's tile (t, w) goes in V's A operand: row tile t, step w / 2,
   // half w % 2, operand lane (4 lg + li % 4, li / 4).
@@ -320,7 +330,7 @@ __device__ __forceinline__ void newton_fwd_chain_body(const T* __restrict__ Mg, 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 16 * t + 4 * lg + r, j = 16 * w + li;
-      if (i < n && j < n) Og[i * n + j] = from_acc<T>(vf[t][r]);
+      if (i < n && j < n) Og[i * n + j] = from_acc<T>(kHalfP * vf[t][r]);
     }
 }
 
@@ -467,7 +477,8 @@ newton_fwd_tile_kernel(const T* __restrict__ mat, T* __restrict__ out, int64_t b
     for (int s = 0; s < KS; ++s) {
       const float4 a = *reinterpret_cast<const float4*>(&Ps[(32 * t + li) * LS + 16 * s + 4 * lh]);
       const float4 b = *reinterpret_cast<const float4*>(&Ps[(32 * t + li) * LS + 16 * s + 8 + 4 * lh]);
-      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      const float x[8] = {kHalfP * a.x, kHalfP * a.y, kHalfP * a.z, kHalfP * a.w,
+                          kHalfP * b.x, kHalfP * b.y, kHalfP * b.z, kHalfP * b.w};
       split8r(x, pa[t][s]);
     }
   // alpha: every wave forms all rows' sums (ascending j, one lane per row).
@@ -491,7 +502,7 @@ newton_fwd_tile_kernel(const T* __restrict__ mat, T* __restrict__ out, int64_t b
   for (int t = 0; t < NR; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      vf[t][r] = alpha * Ps[(32 * t + 8 * (r >> 2) + 4 * lh + (r & 3)) * LS + 32 * w + li];
+      vf[t][r] = twice_v0(alpha, Ps[(32 * t + 8 * (r >> 2) + 4 * lh + (r & 3)) * LS + 32 * w + li]);
       ua[t][r] = vf[t][r];  // the first update: V = 2V - V
     }
   __syncthreads();
@@ -581,7 +592,7 @@ newton_fwd_tile_kernel(const T* __restrict__ mat, T* __restrict__ out, int64_t b
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int i = 32 * t + 8 * (r >> 2) + 4 * lh + (r & 3), j = 32 * w + li;
-      if (i < n && j < n && m0 < bh) Og[i * n + j] = from_acc<T>(2.0f * vf[t][r] - ua[t][r]);
+      if (i < n && j < n && m0 < bh) Og[i * n + j] = from_acc<T>(kHalfP * (2.0f * vf[t][r] - ua[t][r]));
     }
 }
 
@@ -737,7 +748,8 @@ newton_fwd_wide_kernel(const T* __restrict__ mat, T* __restrict__ out, int n, in
     const int t = i / KS, s = i % KS;
     const float4 a = *reinterpret_cast<const float4*>(&Ps[(32 * t + li) * LS + 16 * s + 4 * lh]);
     const float4 b = *reinterpret_cast<const float4*>(&Ps[(32 * t + li) * LS + 16 * s + 8 + 4 * lh]);
-    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    const float x[8] = {kHalfP * a.x, kHalfP * a.y, kHalfP * a.z, kHalfP * a.w,
+                        kHalfP * b.x, kHalfP * b.y, kHalfP * b.z, kHalfP * b.w};
     uint4 h[3];
     split8r(x, h);
     if (i >= L::P3) p3[i >= L::P3 ? i - L::P3 : 0] = h[2];
@@ -756,7 +768,7 @@ newton_fwd_wide_kernel(const T* __restrict__ mat, T* __restrict__ out, int n, in
     float v0[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-      v0[r] = alpha * Ps[(32 * t + 8 * (r >> 2) + 4 * lh + (r & 3)) * LS + 32 * w + li];
+      v0[r] = twice_v0(alpha, Ps[(32 * t + 8 * (r >> 2) + 4 * lh + (r & 3)) * LS + 32 * w + li]);
 #pragma unroll
     for (int k = 0; k < 16; ++k) sp.stage(k, v0, vh[t]);
     if (t == NR - 1)
@@ -852,7 +864,7 @@ newton_fwd_wide_kernel(const T* __restrict__ mat, T* __restrict__ out, int n, in
       // (The last tile's last update is still to be done.)
       const float v = t == NR - 1 ? 2.0f * sp.y[r % 4] - acc[t & 1][r] : sp.y[r % 4];
       const int i = 32 * t + 8 * (r >> 2) + 4 * lh + (r & 3), j = 32 * w + li;
-      if (i < n && j < n) Og[i * n + j] = from_acc<T>(v);
+      if (i < n && j < n) Og[i * n + j] = from_acc<T>(kHalfP * v);
     }
 }
 

@@ -359,6 +359,31 @@ def test_newton_forward_split_nonfinite(gpu, bh, n):
     assert torch.equal(got[2:], good[2:])
 
 
+@pytest.mark.parametrize("bh,n", [(3, 16), (3, 30), (771, 30), (3, 40), (3, 64), (600, 64), (3, 100), (3, 128)])
+def test_newton_forward_range(gpu, bh, n):
+    """The largest finite entries (above the largest bf16) and a huge matrix: alpha underflows to 0
+    and every iterate is 0, no infinity or NaN; without an iteration alpha P itself, its
+    infinities included. The other matrices of the batch are untouched."""
+    import laplacianformer_amd as lf
+
+    print(f"newton forward range bh={bh} n={n}", flush=True)
+    A = torch.from_numpy(gram(bh, n, 64, seed=960 + n)).float().reshape(bh, 1, n, n)
+    big = A.clone()
+    big[0, 0, 1, n - 2] = torch.finfo(torch.float32).max
+    big[1] *= 2.0 ** 126
+    good, got = torch.empty_like(A, device=gpu), torch.empty_like(A, device=gpu)
+    lf.ext().NewtonInverse_forward(A.to(gpu), good, 7)
+    lf.ext().NewtonInverse_forward(big.to(gpu), got, 7)
+    assert not got[:2].any() and torch.equal(got[2:], good[2:]) and bh > 2
+    big = A.clone()
+    big[0, 0, 2, 3] = float("-inf")
+    lf.ext().NewtonInverse_forward(big.to(gpu), got, 0)
+    ref = oracle.newton_forward(big, 0, "f32")
+    assert ref[0, 0, 2, 3] == -np.inf and got[0, 0, 2, 3].item() == -np.inf
+    ref[0, 0, 2, 3] = got[0, 0, 2, 3] = 0.0
+    assert_newton_close(got, ref, "f32", f"n={n} it=0")
+
+
 @pytest.mark.parametrize("bh,n", [(64, 256), (65, 196), (3, 193), (9, 150)])
 def test_newton_large_split(gpu, bh, n):
     """The piece products of n > 128 on both tile sizes (128 x 128 where they give every CU one),
