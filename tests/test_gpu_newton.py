@@ -399,3 +399,49 @@ def test_newton_large_split(gpu, bh, n):
     V, G = gen((bh, 1, n, n), 972 + n, "f32", scale=0.3), gen((bh, 1, n, n), 973 + n, "f32")
     lf.ext().NewtonInverse_backward(G.to(gpu), V.to(gpu), out)
     assert_newton_close(out, oracle.newton_backward(G, V, "f32"), "f32", f"bwd bh={bh} n={n}", rtol=1e-5)
+
+
+@pytest.mark.parametrize("bh,n", [(64, 256), (3, 192), (3, 150)])
+@pytest.mark.parametrize("ev,eg", [(0, -120), (0, -146), (0, 127), (60, 7), (-60, -10), (-130, 120), (80, -140)])
+def test_newton_large_backward_range(gpu, bh, n, ev, eg):
+    """n > 128: inverses and gradients of any magnitude (V ~ 2^ev, G ~ 2^eg; another batch entry
+    stays of order 1) give what the fp64 products give wherever that is a float: the pieces
+    hold no subnormal tail and no infinity of their own."""
+    import laplacianformer_amd as lf
+
+    print(f"newton large backward range bh={bh} n={n} ev={ev} eg={eg}", flush=True)
+    V, G = gen((bh, 1, n, n), 982 + n, "f32", scale=0.05), gen((bh, 1, n, n), 983 + n, "f32", scale=0.1)
+    V[1:], G[1:] = torch.ldexp(V[1:], torch.tensor(ev)), torch.ldexp(G[1:].clamp(-1, 1), torch.tensor(eg))
+    out = torch.full_like(V, float("nan"), device=gpu)
+    lf.ext().NewtonInverse_backward(G.to(gpu), V.to(gpu), out)
+    v64, g64 = V[:3, 0].double(), G[:3, 0].double()
+    ref = -(v64.mT @ g64 @ v64.mT)
+    got = out[:3, 0].cpu().double()
+    assert torch.isfinite(got).all()
+    for i in range(3):
+        # 1e-5 of the largest entry, as elsewhere, and half a subnormal unit at the store.
+        lim = 1e-5 * ref[i].abs().max() + 2.0 ** -150
+        assert ((got[i] - ref[i]).abs() <= lim).all(), (i, ((got[i] - ref[i]).abs().max() / ref[i].abs().max()).item())
+
+
+@pytest.mark.parametrize("bh,n", [(64, 256), (3, 192), (3, 150)])
+@pytest.mark.parametrize("ev,eg", [(0, -120), (0, -146), (0, 127), (60, 7), (-95, 80), (-100, 120), (40, -140)])
+def test_newton_large_backward_range(gpu, bh, n, ev, eg):
+    """n > 128: inverses and gradients of any magnitude (V ~ 2^ev, G ~ 2^eg in all but the first
+    matrix) keep fp32 accuracy: the pieces lose no low bits and no finite entry."""
+    import laplacianformer_amd as lf
+
+    print(f"newton large backward range bh={bh} n={n} ev={ev} eg={eg}", flush=True)
+    V, G = gen((bh, 1, n, n), 982 + n, "f32", scale=0.05), gen((bh, 1, n, n), 983 + n, "f32", scale=0.1)
+    V[1:], G[1:] = torch.ldexp(V[1:], torch.tensor(ev)), torch.ldexp(G[1:].clamp(-1, 1), torch.tensor(eg))
+    out = torch.full_like(V, float("nan"), device=gpu)
+    lf.ext().NewtonInverse_backward(G.to(gpu), V.to(gpu), out)
+    v64, g64 = V[:3, 0].double(), G[:3, 0].double()
+    ref = -(v64.mT @ g64 @ v64.mT)
+    got = out[:3, 0].cpu().double()
+    assert torch.isfinite(got).all()
+    for i in range(3):
+        # 1e-5 of the largest entry, as elsewhere; S = V^T G is an fp32 tensor, whose subnormals
+        # end at 2^-149: half a unit per term of the second sum.
+        lim = 1e-5 * ref[i].abs().max() + 2.0 ** -150 * v64[i].abs().sum(1).max()
+        assert ((got[i] - ref[i]).abs() <= lim).all(), (i, ((got[i] - ref[i]).abs().max() / ref[i].abs().max()).item())
