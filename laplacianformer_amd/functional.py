@@ -86,9 +86,11 @@ class LaplaceKernelFunction(torch.autograd.Function):
         grad = grad.contiguous().to(kern.dtype)
         dq = torch.empty_like(query) if need_q else None
         dk = torch.empty_like(key) if need_k else None
-        if kern.dtype == torch.float32 and ext().LaplaceKernel_backward(grad, kern, query, key, dq, dk, ctx.scale):
-            return dq, dk, None
-        if kern.dtype == torch.float32 and need_q and need_k \
+        # One fused entry per type: the other would allocate its workspace only to refuse.
+        if query.dtype == torch.float16:
+            if ext().LaplaceKernel_backward(grad, kern, query, key, dq, dk, ctx.scale):
+                return dq, dk, None
+        elif kern.dtype == torch.float32 and need_q and need_k \
                 and ext().LaplaceKernel_backward_rows(grad, kern, query, key, dq, dk, ctx.scale):
             return dq, dk, None
         acc = kern.dtype

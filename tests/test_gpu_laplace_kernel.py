@@ -346,6 +346,24 @@ def test_kernel_backward_rows(gpu, dt, lens, bh, M, C):
     assert_l1_close(dk, rk, dt, "dk (sum over the sets)", np.broadcast_to(scale, rk.shape))
 
 
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("B,N,M,C", [(300, 9, 49, 64), (4, 196, 49, 64), (2, 70, 100, 64)])
+def test_kernel_backward_allocations(gpu, dt, B, N, M, C):
+    """The kernel's backward allocates the two gradients and one workspace."""
+    from laplacianformer_amd.functional import LaplaceKernelFunction
+
+    print(f"laplace kernel backward allocations {dt} B={B} N={N} M={M} C={C}", flush=True)
+    q = gen((B, 1, N, C), 921, dt).to(gpu).requires_grad_()
+    k = gen((B, 1, C, M), 922, dt).to(gpu).requires_grad_()
+    gk = gen((B, 1, N, M), 923, "f32").to(gpu)
+    kern = LaplaceKernelFunction.apply(q, k, 0.125)
+    torch.cuda.synchronize()
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]  # noqa: E731
+    before = count()
+    torch.autograd.grad(kern, (q, k), gk)
+    assert count() - before <= 3
+
+
 @pytest.mark.parametrize("M,C", [(49, 64), (16, 20), (196, 64)])
 @pytest.mark.parametrize("keys", ["subnormal", "huge", "inf"])
 def test_f32_step_range(gpu, M, C, keys):
