@@ -2256,6 +2256,10 @@ int rows_bwd_dims(int dtype, int nsrc, const int64_t* lens, Dims& d, const char*
                 (long long)d.C);
   return LFAMD_OK;
 }
+
+// The register-column kernel's partial sums; 16 bytes, for a size that is not 0, where a
+// slice's only workgroup stores grad_key itself and none are written.
+size_t rows_bwd_bytes(const BcPlan& p) { return p.nx == 1 ? 16 : p.partialElems * 4; }
 }  // namespace
 
 size_t lfamd_laplace_kernel_backward_rows_workspace_size(int dtype, int num_sources, const int64_t* q_lens,
@@ -2264,7 +2268,7 @@ size_t lfamd_laplace_kernel_backward_rows_workspace_size(int dtype, int num_sour
   const char* who = "laplace kernel backward (row sets)";
   Dims d{batch, heads, 1, k_len, channels};
   if (!valid_dtype(dtype) || check_dims(d, who) || rows_bwd_dims(dtype, num_sources, q_lens, d, who)) return 0;
-  return (kernel_bwd_bcast(dtype, d) ? plan_bcast(d, true).partialElems : plan_mb(d, true).partialElems) * 4;
+  return kernel_bwd_bcast(dtype, d) ? rows_bwd_bytes(plan_bcast(d, true)) : plan_mb(d, true).partialElems * 4;
 }
 
 int lfamd_laplace_kernel_backward_rows(int dtype, int num_sources, const float* const* grad_kernels,
@@ -2289,7 +2293,7 @@ int lfamd_laplace_kernel_backward_rows(int dtype, int num_sources, const float* 
                                 bcast ? 1 : kMbRB, scale);
   const BcPlan bp = bcast ? plan_bcast(d, true) : BcPlan{};
   const MbPlan mp = bcast ? MbPlan{} : plan_mb(d, true);
-  const size_t need = (bcast ? bp.partialElems : mp.partialElems) * 4;
+  const size_t need = bcast ? rows_bwd_bytes(bp) : mp.partialElems * 4;
   if (!workspace || workspace_bytes < need)
     return fail(LFAMD_ERR_ARG, "%s: workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
   return bcast ? launch_bcast_bwd<true, true, kGradKernel>(dtype, nullptr, nullptr, key, nullptr, grad_key, workspace,

@@ -349,7 +349,10 @@ def test_kernel_backward_rows(gpu, dt, lens, bh, M, C):
 @pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("B,N,M,C", [(300, 9, 49, 64), (4, 196, 49, 64), (2, 70, 100, 64)])
 def test_kernel_backward_allocations(gpu, dt, B, N, M, C):
-    """The kernel's backward allocates the two gradients and one workspace."""
+    """The kernel's backward allocates the two gradients and one workspace, which holds partial
+    sums only where a slice has several workgroups (300 slices of 9 rows on the register-column
+    kernel have one each and store grad_key themselves)."""
+    import laplacianformer_amd as lf
     from laplacianformer_amd.functional import LaplaceKernelFunction
 
     print(f"laplace kernel backward allocations {dt} B={B} N={N} M={M} C={C}", flush=True)
@@ -362,6 +365,12 @@ def test_kernel_backward_allocations(gpu, dt, B, N, M, C):
     before = count()
     torch.autograd.grad(kern, (q, k), gk)
     assert count() - before <= 3
+    if B == 300 and dt != "f16":
+        import ctypes
+
+        one = (ctypes.c_int64 * 1)(N)
+        code = lf.dtype_code(q)
+        assert lf.capi().lfamd_laplace_kernel_backward_rows_workspace_size(code, 1, one, B, 1, M, C) == 16
 
 
 @pytest.mark.parametrize("M,C", [(49, 64), (16, 20), (196, 64)])
