@@ -686,6 +686,20 @@ constexpr int kBcBufs = 4;  // LDS accumulators of the workgroup grad_key reduct
 // unscaled step alone.
 constexpr float kStepKeyMax = 0x1p103f, kStepPre = 0x1p24f, kStepFast = 0x1p126f, kStepSlow = 0x1p100f;
 
+// f(column, channel) over a 64-channel tile of MC columns, consecutive lanes on consecutive
+// columns (contiguous in the key's layout) and consecutive passes on consecutive channels.
+// 64 / MC channels a pass, so no division; the loop stays short, since what a call of a few
+// rows pays for here is fetching its instructions once (with t / MC and t % MC of one flat
+// loop, one row, fp32, M = 49, C = 64, grad_key: 19.7 us, now 11.3; before that loop 13.8).
+template <int MC, typename F> __device__ __forceinline__ void each_tile_column(int W, int wave, int lane, F f) {
+  constexpr int CP = 64 / MC;
+  static_assert(CP == 1 || CP * MC == 64, "whole channels per pass");
+  const int j = CP == 1 ? lane : lane % MC;
+  if (j < MC)
+#pragma unroll 4
+    for (int cl = wave * CP + (CP == 1 ? 0 : lane / MC); cl < 64; cl += W * CP) f(j, cl);
+}
+
 // Floats of the key tile [mc][65], whole 16-byte groups.
 __host__ __device__ constexpr int bcast_key_floats(int mc) { return (mc * 65 + 3) & ~3; }
 
@@ -718,12 +732,15 @@ __device__ __forceinline__ void bcast_reduce_dk(const float (&v)[MC], float* red
     }
     __syncthreads();
   }
-  for (int t = threadIdx.x; t < 64 * MC; t += blockDim.x) {
-    const int j = cols ? t % MC : t >> 6, cl = cols ? t / MC : t & 63;
+  auto sum = [&](int j, int cl) {
     float s = red[j * 65 + cl];
     for (int b = 1; b < nb; ++b) s += red[b * BF + j * 65 + cl];
-    out(j, cl, s);
-  }
+    return s;
+  };
+  if (cols)
+    each_tile_column<MC>(W, wave, lane, [&](int j, int cl) { out(j, cl, sum(j, cl)); });
+  else
+    for (int j = wave; j < MC; j += W) out(j, lane, sum(j, lane));
 }
 
 __host__ __device__ constexpr int bcast_max_waves(int mc) { return mc <= 16 ? 16 : 12; }
@@ -739,6 +756,13 @@ enum BwdGrad { kGradF16 = 0, kGradKernel = 1 };
 // Whether a backward kernel compiles both fp32 step loops (kStepFast).
 template <typename T, bool DQ, bool DK, int GSRC>
 constexpr bool two_step_loops() { return sizeof(T) == 4 && !(DQ && DK) && GSRC == kGradF16; }
+
+// fp32 grad_query alone, a row per wave: two workgroups fit a CU (64 registers at M = 16, 128 at
+// M = 49), which counts where the slices outnumber the CUs. Both step loops take 73 and 134
+// registers: M = 49 is held to its 128, M = 16 keeps the one loop (300 slices of 100 rows, M = 16,
+// C = 64: 11.2 us with both loops, now 9.7).
+template <typename T, int MC, bool DQ, bool DK, int GSRC, int RPW>
+constexpr bool bcast_paired() { return two_step_loops<T, DQ, DK, GSRC>() && !DK && RPW == 1; }
 
 // The kernel-gradient backward's rows: up to three row sets (a layer's K_mm, K_qm and
 // K_km share one key) taken as one concatenation, set i ending at row (column-block
@@ -768,9 +792,10 @@ __device__ __forceinline__ P pick3(const P (&a)[3], int s) {
 
 // RPW = 2 (C <= 32): a wave's halves take two rows at once, lane (h, c) channel c of
 // row 2i + h, where one row would leave half the lanes idle; the halves' grad_key sums
-// are added at the end.
+// are added at the end. (M = 49 with grad_key: 4 to 13 registers spill in this form, 11 to
+// 13 with both gradients of a kernel gradient; 3 of that one's with RPW = 1.)
 template <typename T, int MC, bool DQ, bool DK, int GSRC = kGradF16, int RPW = 1>
-__global__ void __launch_bounds__(64 * bcast_max_waves(MC))
+__global__ void __launch_bounds__(64 * bcast_max_waves(MC), (bcast_paired<T, MC, DQ, DK, GSRC, RPW>() ? (MC <= 16 ? 8 : 4) : 1))
 laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscale, const T* __restrict__ query,
                          const T* __restrict__ key, T* __restrict__ dq, T* __restrict__ dk,
                          float* __restrict__ partial, int N, int C, int rowsPerWave) {
@@ -779,7 +804,7 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscal
   constexpr bool kF16 = std::is_same<T, f16s>::value;
   // 16-bit inputs take the ordered-pattern step (tmap16): y = clamp(T(q) + (1/2 - T(k))).
   constexpr bool k16 = sizeof(T) == 2;
-  constexpr bool kTwo = two_step_loops<T, DQ, DK, GSRC>();
+  constexpr bool kTwo = two_step_loops<T, DQ, DK, GSRC>() && !(MC <= 16 && bcast_paired<T, MC, DQ, DK, GSRC, RPW>());
   constexpr int EPW = sizeof(T) == 2 ? 2 : 1;    // grad elements per 32-bit word
   constexpr int GD = GSRC == kGradF16 ? RB * MC / EPW : RB * MC;  // grad words of a full batch
   constexpr int NL = (GD + 63) / 64;             // words per lane per batch
@@ -863,8 +888,7 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscal
   // Key tile (contiguous reads; the pitch of 65 spreads the stores over the banks): 16-bit
   // keys as the step terms 1/2 - T(k), fp32 keys as values.
   bool big = false;
-  for (int t = threadIdx.x; t < 64 * MC; t += blockDim.x) {
-    const int cl = t / MC, j = t - cl * MC;
+  each_tile_column<MC>(W, wave, lane, [&](int j, int cl) {
     const int cc = cb * 64 + cl;
     const T kv = kb[(size_t)min(cc, C - 1) * MC + j];
     float v;
@@ -872,7 +896,7 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscal
     else v = to_acc(kv);
     if constexpr (kTwo) big |= !(fabsf(v) < kStepKeyMax);
     ksm[j * 65 + cl] = cc < C ? v : 0.0f;
-  }
+  });
   bool fast = false;  // (workgroup-uniform)
   if constexpr (kTwo) fast = !__syncthreads_or(big);
   else __syncthreads();
@@ -946,11 +970,11 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscal
       // the additions, so no chain of dependent LDS round trips.
       if (DQ) {
         const float4* rowp = reinterpret_cast<const float4*>(gsm + min(lane, RB - 1) * MP);
-        // (Half the row at a time: a whole row's registers would spill some of the columns'.)
-        constexpr int HQ = MP / 8;
+        // (M = 49: half the row at a time, a whole row's registers would spill some of the columns'.)
+        constexpr int NH = MC > 32 ? 2 : 1, HQ = MP / 4 / NH;
         float sum = 0.0f;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < NH; ++h) {
           float4 v[HQ];
 #pragma unroll
           for (int jq = 0; jq < HQ; ++jq) v[jq] = rowp[h * HQ + jq];
@@ -1094,7 +1118,9 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscal
 constexpr int kMbMC = 32;  // columns per wave
 constexpr int kMbRB = 8;   // rows per batch
 
-template <typename T, int CB, bool DQ, bool DK, int GSRC = kGradF16>
+// LOOP: a batch's rows go through a loop, only those there are, with the one fp32 step; otherwise
+// the batch is unrolled (below). mb_row_loop says which.
+template <typename T, int CB, bool DQ, bool DK, int GSRC = kGradF16, bool LOOP = false>
 __global__ void __launch_bounds__(1024)
 laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, const T* __restrict__ key,
                       T* __restrict__ dq, float* __restrict__ partial, int N, int C, int rowsPerWG, int Mt,
@@ -1106,7 +1132,7 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
   constexpr int MP = MC;                       // LDS row pitch of a staged batch (floats)
   // 16-bit inputs take the ordered-pattern step (tmap16): y = clamp(T(q) + (1/2 - T(k))).
   constexpr bool k16 = std::is_same<T, f16s>::value || std::is_same<T, bf16s>::value;
-  constexpr bool kTwo = two_step_loops<T, DQ, DK, GSRC>();
+  constexpr bool kTwo = !LOOP && two_step_loops<T, DQ, DK, GSRC>();
   // Grad elements per fetched 32-bit word: 2 for 16-bit grads, 1 for fp32 grads and
   // for the kernel-gradient source (fp32 gK and K, g = -s * gK * K formed at staging).
   constexpr int EPW = GSRC == kGradKernel ? 1 : (4 / (int)sizeof(T) > 0 ? 4 / (int)sizeof(T) : 1);
@@ -1294,45 +1320,73 @@ laplace_bwd_mb_kernel(const T* __restrict__ gout, const T* __restrict__ query, c
         float4 gq[LA];
 #pragma unroll
         for (int u = 0; u < LA; ++u) gq[u] = g4[u];
-        unrolled<RB>([&](auto rc) {
-          constexpr int r = rc.value;
-          const float qv = qn;
-          float acc[4] = {accn, 0.0f, 0.0f, 0.0f};
-          unrolled<NQ>([&](auto jc) {
-            constexpr int jq = jc.value, at = r * NQ + jq;
-            const float4 gv = gq[at % LA];
-            if constexpr (at + LA < NG) gq[at % LA] = g4[at + LA];
-            if constexpr (jq == NQ - 1 && r + 1 < RB) {
-              qn = qsm[(r + 1) * 64 + lane];
-              if (DQ) accn = gneg[r + 1];
-            }
-            const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
+        auto columns = [&](auto jc, float4 gv, float qv, float (&acc)[4]) {
+          const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int j = jq * 4 + u;
-              float y;
-              if constexpr (k16) {
-                y = __builtin_amdgcn_fmed3f(qv + kreg[j], 0.0f, 1.0f);  // one clamped add
-              } else if constexpr (decltype(fastc)::value) {
-                y = __builtin_amdgcn_fmed3f(__builtin_fmaf(qv - kreg[j], scl, 0.5f), 0.0f, 1.0f);
-              } else {
-                const float e = (qv - kreg[j]) * scl;
-                y = __builtin_amdgcn_fmed3f(__builtin_fmaf(e, scl, 0.5f), 0.0f, 1.0f);
-              }
-              if (DQ) acc[u] = fmaf(gg[u], y, acc[u]);
-              if (DK) {
-                dka[j] = fmaf(gg[u], y, dka[j]);
-                asm volatile("" : "+v"(dka[j]));  // update in place, not after the row
-              }
+          for (int u = 0; u < 4; ++u) {
+            const int j = decltype(jc)::value * 4 + u;
+            float y;
+            if constexpr (k16) {
+              y = __builtin_amdgcn_fmed3f(qv + kreg[j], 0.0f, 1.0f);  // one clamped add
+            } else if constexpr (decltype(fastc)::value) {
+              y = __builtin_amdgcn_fmed3f(__builtin_fmaf(qv - kreg[j], scl, 0.5f), 0.0f, 1.0f);
+            } else {
+              const float e = (qv - kreg[j]) * scl;
+              y = __builtin_amdgcn_fmed3f(__builtin_fmaf(e, scl, 0.5f), 0.0f, 1.0f);
             }
-            __builtin_amdgcn_sched_barrier(0);
-          });
+            if (DQ) acc[u] = fmaf(gg[u], y, acc[u]);
+            if (DK) {
+              dka[j] = fmaf(gg[u], y, dka[j]);
+              asm volatile("" : "+v"(dka[j]));  // update in place, not after the row
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        auto store_row = [&](int r, const float (&acc)[4]) {
           if (DQ) {
             float total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
             asm volatile("" : "+v"(total));
             dqp[r * 64 + lane] = total;
           }
-        });
+        };
+        if constexpr (LOOP) {
+#pragma unroll 1
+          for (int r = 0; r < nr; ++r) {
+            const int rn = min(r + 1, RB - 1);
+            const float4* gr = g4 + r * NQ;
+            const float4* gn = g4 + rn * NQ;
+            const float qv = qn;
+            float acc[4] = {accn, 0.0f, 0.0f, 0.0f};
+            unrolled<NQ>([&](auto jc) {
+              constexpr int jq = jc.value;
+              const float4 gv = gq[jq % LA];
+              gq[jq % LA] = jq + LA < NQ ? gr[jq + LA] : gn[jq + LA - NQ];
+              if constexpr (jq == NQ - 1) {
+                qn = qsm[rn * 64 + lane];
+                if (DQ) accn = gneg[rn];
+              }
+              columns(jc, gv, qv, acc);
+            });
+            store_row(r, acc);
+          }
+        } else {
+          unrolled<RB>([&](auto rc) {
+            constexpr int r = rc.value;
+            const float qv = qn;
+            float acc[4] = {accn, 0.0f, 0.0f, 0.0f};
+            unrolled<NQ>([&](auto jc) {
+              constexpr int jq = jc.value, at = r * NQ + jq;
+              const float4 gv = gq[at % LA];
+              if constexpr (at + LA < NG) gq[at % LA] = g4[at + LA];
+              if constexpr (jq == NQ - 1 && r + 1 < RB) {
+                qn = qsm[(r + 1) * 64 + lane];
+                if (DQ) accn = gneg[r + 1];
+              }
+              columns(jc, gv, qv, acc);
+            });
+            store_row(r, acc);
+          });
+        }
       }
       if (DQ) {
         // Every wave of the workgroup has written this batch's partials (and is
@@ -1826,10 +1880,28 @@ MbPlan plan_mb(const Dims& d, bool dkey) {
   return p;
 }
 
+// Rows through a loop (LOOP) instead of an unrolled batch of eight, which computes a short
+// batch's missing rows too (on zero grad) and whose instructions a few rows do not pay back:
+//   up to 6 rows (fp32 grad_query, one row, M = 32: 4.6 us against 6.4 unrolled; five rows 6.1
+//   against 6.8);
+//   where three waves or more per SIMD have rows, so that issue slots count, and the missing rows
+//   cost more than the loop: 2, 3, 8 % of the rows for grad_key, grad_query, both, 50 % for both of
+//   a kernel gradient, whose loop spills (bf16 grad_query, C = 64: 2048 slices of 9 rows, M = 196, 90
+//   against 98 us; 4 of 17 rows, M = 196, 14.7 against 15.6; 256 of 130 rows, M = 17, 11.3 against
+//   12.0; fp16 kernel gradient, 64 slices of 50 rows, M = 64, 18.2 looped against 17.4).
+// Full batches are faster unrolled at any count (fp32 grad_query, 300 slices of 64 rows, M = 64:
+// 0.9 of the loop's time). Several workgroups per slice: only the last can have a short batch.
+bool mb_row_loop(const Dims& d, const MbPlan& p, bool dq, bool dk, int gsrc) {
+  if (p.nx > 1 || d.N < 1) return false;
+  const int64_t padded = (d.N + kMbRB - 1) / kMbRB * kMbRB;
+  const int percent = gsrc == kGradKernel ? 50 : dq && dk ? 8 : dq ? 3 : 2;
+  return d.N <= 6 || (padded / kMbRB * p.CB >= 12 && 100 * padded > (100 + percent) * d.N);
+}
+
 template <typename T, int CB, bool DQ, bool DK, int GSRC = kGradF16>
 int launch_mb_cb(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
                  const MbPlan& p, hipStream_t st, const KernGrad& kg = {}) {
-  auto kern = laplace_bwd_mb_kernel<T, CB, DQ, DK, GSRC>;
+  auto kern = mb_row_loop(d, p, DQ, DK, GSRC) ? laplace_bwd_mb_kernel<T, CB, DQ, DK, GSRC, true> : laplace_bwd_mb_kernel<T, CB, DQ, DK, GSRC>;
   if (p.lds > 65536)
     if (int s = set_dyn_lds(reinterpret_cast<const void*>(kern), p.lds, "laplace backward")) return s;
   dim3 grid(p.nx, p.ncb, (unsigned)d.BH());

@@ -296,7 +296,8 @@ def test_kernel_forward_multi_rejects(gpu):
                                          ((196, 196, 49), (32, 8), 49, 32), ((33, 130), (1, 2), 49, 96),
                                          ((16, 65, 9), (1, 2), 16, 31), ((64, 129, 3), (1, 2), 32, 64),
                                          ((50, 71, 8), (1, 2), 50, 40), ((196, 333, 1), (1, 2), 196, 64),
-                                         ((17,), (1, 1), 255, 65)],
+                                         ((17,), (1, 1), 255, 65), ((3,), (2, 1), 100, 64), ((9,), (3, 1), 196, 40),
+                                         ((1, 1), (1, 2), 49, 64), ((5,), (1, 2), 16, 64)],
                          ids=lambda s: "-".join(map(str, s)) if isinstance(s, tuple) else str(s))
 def test_kernel_backward_rows(gpu, dt, lens, bh, M, C):
     """lfamd_laplace_kernel_backward_rows: up to three row sets against one key in one launch, every
