@@ -21,6 +21,18 @@ def test_profiled_kernel_names_are_in_the_summaries():
         assert name in counters, f"{name} is not in profiles/laplace_newton_counters.json"
 
 
+def test_profiled_kernels_are_in_the_library(tmp_path):
+    """The kernels whose counters the bench line prints beside its times are ones that the built
+    library still has: the summaries keep the names of what ran when they were made."""
+    import bench
+    import test_kernel_resources_cpu as resources
+
+    names = subprocess.run(["c++filt"], input="\n".join(k["name"] for k in resources._gfx950_kernels(resources.LIB, tmp_path)),
+                           capture_output=True, text=True, check=True).stdout.splitlines()
+    for name in [bench.K_FWD, bench.K_BWD, bench.K_RED, bench.K_NF, bench.K_NB]:
+        assert any(n.removeprefix("void ").startswith(name + "(") for n in names), f"{name} is not in the built library"
+
+
 def test_more_than_one_gpu_is_refused():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True,
                        text=True, timeout=120)
