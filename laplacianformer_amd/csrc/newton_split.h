@@ -686,8 +686,8 @@ template <int NR, int KS> struct WideLayout {
 // instructions, since each SIMD has one wave: beside the products of row tile t run
 // the split of T's tile t - 1 (or V's update) and the storing of V's tile t. 512 x 100^2, 10 iterations: 168 us against 272 with fp32
 // matrix instructions, 64 x 100^2 82 against 130, 1024 x 128^2, 12 iterations, 647
-// against 997 (KS = 8 spills some of P's third pieces: 384 registers are allowed, 256
-// and 128 accumulation ones).
+// against 997 (NR = 4 spills P's third pieces, 38 registers at KS = 7, the n = 100 above
+// among them, and 185 at KS = 8: 384 are allowed, 256 and 128 accumulation ones).
 template <typename T, int NR, int KS>
 __global__ void __launch_bounds__(64 * NR) __attribute__((amdgpu_waves_per_eu(1, 1), amdgpu_num_vgpr(192)))
 newton_fwd_wide_kernel(const T* __restrict__ mat, T* __restrict__ out, int n, int iters) {
