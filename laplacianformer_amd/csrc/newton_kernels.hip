@@ -1443,23 +1443,29 @@ template <int NP> constexpr int narrow_wpr() { return pick_wpr<NP>() == 4 ? 2 : 
 // it is), or too few for the pieces' set-up and their one workgroup per matrix:
 //   n <= 32    up to two matrices per CU, whose two waves have nothing to hide the splitting
 //              behind (512 x 32^2, 12 iterations 12.1 against 14.9 us, 8 matrices 9.7 / 10.5;
-//              600 15.6 / 15.0, 1024 18.7 / 16.4), and two iterations (1024, one: 5.5 / 5.7);
-//   49 .. 64   one iteration (bf16 512 x 64^2 9.8 against 12.4 us), two below two matrices
-//              per CU (8 matrices 7.9 / 8.4; 512 x 64^2 14.4 / 11.6);
-//   65 .. 96   two iterations above one matrix per CU, where several of this kernel share one
-//              (512 x 80^2: one 22.6 against 27.1 us, two 32.8 / 35.0, three 42.7 / 41.6);
+//              600 15.6 / 15.0, 1024 18.7 / 16.4), up to three for six iterations (600 x 24^2,
+//              three 7.9 / 8.3), and two iterations (1024, one: 5.5 / 5.7);
+//   49 .. 64   one iteration (bf16 512 x 64^2 9.8 against 12.4 us), two as well (bf16 512 x 64^2
+//              15.5 / 16.5; 8 matrices 7.9 / 8.4) but for whole fp32 tiles from two matrices
+//              per CU on (512 x 64^2 14.4 / 11.6);
+//   65 .. 112  one iteration (bf16 8 x 96^2 15.2 / 16.2), above one matrix per CU, where several
+//              of this kernel share one, two up to n = 96 (512 x 80^2: one 22.6 against 27.1 us, two
+//              32.8 / 35.0) and three up to n = 80 (bf16 512 x 80^2 43.4 / 46.5);
 //   113 .. 128 two iterations, three above 64 matrices, four from one per CU on: the wide
 //              kernel's spilled third pieces cost 20 to 50 us a call (256 x 128^2: one 26.7 against
 //              67.4 us, four 73.6 / 94.2, six about 106 / 114; 128 matrices, three, 57 / 71).
-// fp32 n = 17 and 65 always: row 16 (64) runs on the VALU beside the strips, where the pieces
-// pad it to a tile (1024 x 17^2, 12 iterations 11.5 against 15.7 us; 512 x 65^2 82.5 / 111).
-template <int NP> bool fwd_on_fp32(int64_t bh, int iters) {
+// fp32 n = 17, 33 and 65 always: row 16 (32, 64) runs on the VALU beside the strips, where the
+// pieces pad it to a tile (1024 x 17^2, 12 iterations 11.5 against 15.7 us; 1024 x 33^2, ten
+// 33.8 / 35.3; 512 x 65^2 82.5 / 111).
+template <typename T, int NP> bool fwd_on_fp32(int64_t bh, int n, int iters) {
   const bool many = fwd_many(bh);
+  const int64_t cus = num_cus();
   if (iters == 0) return true;
-  if (NP == 32) return iters <= 2 || bh <= 2 * (int64_t)num_cus();
-  if (NP == 64) return iters <= (many ? 1 : 2);
-  if (NP == 80 || NP == 96) return iters <= 2 && bh > num_cus();
-  if (NP == 128) return iters <= (bh >= num_cus() ? 4 : bh > num_cus() / 4 ? 3 : 2);
+  if (NP == 32) return iters <= 2 || bh <= 2 * cus || (bh <= 3 * cus && iters <= 6);
+  if (NP == 64) return iters <= (many && std::is_same<T, float>::value && n == NP ? 1 : 2);
+  if (NP == 80 || NP == 96) return iters <= (bh > cus ? (NP == 80 ? 3 : 2) : 1);
+  if (NP == 112) return iters <= 1;
+  if (NP == 128) return iters <= (bh >= cus ? 4 : bh > cus / 4 ? 3 : 2);
   return false;
 }
 
@@ -1481,9 +1487,9 @@ int fwd_np(const T* m, T* o, int64_t bh, int n, int iters, hipStream_t st) {
     if (n == 49)
       return many ? launch_fwd(newton_fwd_sym_kernel<8>, bh, 512, fwd_lds<NP>(), st, m, o, n, iters)
                   : launch_fwd(newton_fwd_sym_kernel<16>, bh, 1024, fwd_lds<NP>(), st, m, o, n, iters);
-  if constexpr (std::is_same<T, float>::value && (NP == 32 || NP == 80))
+  if constexpr (std::is_same<T, float>::value && (NP == 32 || NP == 48 || NP == 80))
     if (n == NP - 15) return fwd_fp32<T, NP, 1>(m, o, bh, n, iters, st);
-  if (NP == 16 || fwd_on_fp32<NP>(bh, iters)) return fwd_fp32<T, NP, 4>(m, o, bh, n, iters, st);
+  if (NP == 16 || fwd_on_fp32<T, NP>(bh, n, iters)) return fwd_fp32<T, NP, 4>(m, o, bh, n, iters, st);
   if constexpr (NP == 16) {
     return LFAMD_OK;  // (not reached: the pieces' kernels have no 16 bucket)
   } else if constexpr (NP <= 64) {
@@ -1705,7 +1711,7 @@ int lfamd_attention_landmarks_forward(const float* kmm, const float* kkm, int v_
   float* part = static_cast<float*>(workspace);
   if (iters < 0) iters = 0;
   if (int s = tall_t_check(v_dtype, kkm, v, workspace_bytes, slices, rows, m, d, &per)) return s;
-  if (m != 49 && (fwd_many(slices) || fwd_on_fp32<64>(slices, iters))) {
+  if (m != 49 && (fwd_many(slices) || fwd_on_fp32<float, 64>(slices, m, iters))) {
     // Two matrices per CU and more, or too few iterations: lfamd_newton_forward's own kernel
     // for them, which no CU has room beside, then the tall product (196 rows, m = 64, 10 iterations: 512 slices 62.2
     // against 70.4 us with the chain body beside the tall product, 1024 102.8 against 127.5,

@@ -327,7 +327,10 @@ def test_newton_forward_split(gpu, bh, n, dt, iters):
                                            (256, 80, "f32", 2), (257, 80, "f16", 2), (257, 90, "bf16", 3),
                                            (2, 105, "bf16", 6), (2, 105, "f16", 0), (2, 128, "f32", 2),
                                            (65, 128, "f32", 3), (64, 128, "f16", 3), (256, 128, "f32", 4),
-                                           (256, 115, "bf16", 5)])
+                                           (256, 115, "bf16", 5), (3, 33, "f32", 6), (513, 33, "f32", 3),
+                                           (3, 33, "bf16", 6), (600, 24, "bf16", 6), (769, 24, "f32", 4),
+                                           (512, 64, "f32", 2), (512, 64, "bf16", 2), (2, 90, "f32", 1),
+                                           (257, 80, "f32", 3), (257, 96, "f32", 3), (2, 105, "bf16", 1)])
 def test_newton_forward_fp32_rule(gpu, bh, n, dt, iters):
     """Both sides of the rule between the fp32 matrix instructions and the bf16 pieces (counts of
     matrices and iterations, n = 17 and 65), on general matrices."""
