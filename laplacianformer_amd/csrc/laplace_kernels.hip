@@ -687,13 +687,14 @@ constexpr int kBcBufs = 4;  // LDS accumulators of the workgroup grad_key reduct
 constexpr float kStepKeyMax = 0x1p103f, kStepPre = 0x1p24f, kStepFast = 0x1p126f, kStepSlow = 0x1p100f;
 
 // f(column, channel) over a 64-channel tile of MC columns, consecutive lanes on consecutive
-// columns (contiguous in the key's layout) and consecutive passes on consecutive channels.
-// 64 / MC channels a pass, so no division; the loop stays short, since what a call of a few
-// rows pays for here is fetching its instructions once (with t / MC and t % MC of one flat
-// loop, one row, fp32, M = 49, C = 64, grad_key: 19.7 us, now 11.3; before that loop 13.8).
+// columns (contiguous in the key's layout), 64 / MC channels per wave and pass, so no division. The loop
+// stays short, since what a call of a few rows pays for here is fetching its instructions once (with t / MC
+// and t % MC of one flat loop, one row, fp32, M = 49, C = 64, grad_key: 19.7 us, now 11.3; before that loop
+// 13.8. Flat for M = 16 and 32 alone: fp16 grad_query, 2048 slices of 9 rows, M = 32, 36.7 against 23 us).
 template <int MC, typename F> __device__ __forceinline__ void each_tile_column(int W, int wave, int lane, F f) {
   constexpr int CP = 64 / MC;
   static_assert(CP == 1 || CP * MC == 64, "whole channels per pass");
+  asm volatile("" : "+v"(lane));  // the lane's place is formed anew, not held in registers through the row loop
   const int j = CP == 1 ? lane : lane % MC;
   if (j < MC)
 #pragma unroll 4
@@ -757,10 +758,10 @@ enum BwdGrad { kGradF16 = 0, kGradKernel = 1 };
 template <typename T, bool DQ, bool DK, int GSRC>
 constexpr bool two_step_loops() { return sizeof(T) == 4 && !(DQ && DK) && GSRC == kGradF16; }
 
-// fp32 grad_query alone, a row per wave: two workgroups fit a CU (64 registers at M = 16, 128 at
-// M = 49), which counts where the slices outnumber the CUs. Both step loops take 73 and 134
-// registers: M = 49 is held to its 128, M = 16 keeps the one loop (300 slices of 100 rows, M = 16,
-// C = 64: 11.2 us with both loops, now 9.7).
+// fp32 grad_query alone, a row per wave: where the slices outnumber the CUs it counts that two
+// workgroups fit one, 128 registers at M = 49 (both step loops took 134), 64 at M = 16 (300 slices of 100
+// rows, C = 64: 9.7 us, 11.2 with the 73 that both loops took). 64 registers hold one loop only: TWO says
+// whether both are compiled (launch_bcast_bwd_rpw).
 template <typename T, int MC, bool DQ, bool DK, int GSRC, int RPW>
 constexpr bool bcast_paired() { return two_step_loops<T, DQ, DK, GSRC>() && !DK && RPW == 1; }
 
@@ -792,10 +793,11 @@ __device__ __forceinline__ P pick3(const P (&a)[3], int s) {
 
 // RPW = 2 (C <= 32): a wave's halves take two rows at once, lane (h, c) channel c of
 // row 2i + h, where one row would leave half the lanes idle; the halves' grad_key sums
-// are added at the end. (M = 49 with grad_key: 4 to 13 registers spill in this form, 11 to
-// 13 with both gradients of a kernel gradient; 3 of that one's with RPW = 1.)
-template <typename T, int MC, bool DQ, bool DK, int GSRC = kGradF16, int RPW = 1>
-__global__ void __launch_bounds__(64 * bcast_max_waves(MC), (bcast_paired<T, MC, DQ, DK, GSRC, RPW>() ? (MC <= 16 ? 8 : 4) : 1))
+// are added at the end. (M = 49 with grad_key: up to 13 registers spill in this form, 11 to 13 with
+// both gradients of a kernel gradient, 3 of that one's and 2 of fp32 grad_key's with RPW = 1.)
+template <typename T, int MC, bool DQ, bool DK, int GSRC = kGradF16, int RPW = 1, bool TWO = true>
+__global__ void __launch_bounds__(64 * bcast_max_waves(MC),
+                                  (bcast_paired<T, MC, DQ, DK, GSRC, RPW>() ? (MC > 16 ? 4 : TWO ? 7 : 8) : 1))
 laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscale, const T* __restrict__ query,
                          const T* __restrict__ key, T* __restrict__ dq, T* __restrict__ dk,
                          float* __restrict__ partial, int N, int C, int rowsPerWave) {
@@ -804,7 +806,7 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscal
   constexpr bool kF16 = std::is_same<T, f16s>::value;
   // 16-bit inputs take the ordered-pattern step (tmap16): y = clamp(T(q) + (1/2 - T(k))).
   constexpr bool k16 = sizeof(T) == 2;
-  constexpr bool kTwo = two_step_loops<T, DQ, DK, GSRC>() && !(MC <= 16 && bcast_paired<T, MC, DQ, DK, GSRC, RPW>());
+  constexpr bool kTwo = TWO && two_step_loops<T, DQ, DK, GSRC>();
   constexpr int EPW = sizeof(T) == 2 ? 2 : 1;    // grad elements per 32-bit word
   constexpr int GD = GSRC == kGradF16 ? RB * MC / EPW : RB * MC;  // grad words of a full batch
   constexpr int NL = (GD + 63) / 64;             // words per lane per batch
@@ -970,8 +972,9 @@ laplace_bwd_bcast_kernel(const T* __restrict__ gout, RowSources src, float gscal
       // the additions, so no chain of dependent LDS round trips.
       if (DQ) {
         const float4* rowp = reinterpret_cast<const float4*>(gsm + min(lane, RB - 1) * MP);
-        // (M = 49: half the row at a time, a whole row's registers would spill some of the columns'.)
-        constexpr int NH = MC > 32 ? 2 : 1, HQ = MP / 4 / NH;
+        // (Half the row at a time: a whole row's registers would spill some of the columns' at M = 49 and
+        // cost a wave per SIMD at M = 32.)
+        constexpr int NH = 2, HQ = MP / 4 / NH;
         float sum = 0.0f;
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
@@ -1809,7 +1812,13 @@ template <typename T, int MC, bool DQ, bool DK, int GSRC, int RPW>
 int launch_bcast_bwd_rpw(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
                          const BcPlan& p, hipStream_t st, const KernGrad& kg) {
   dim3 grid(p.nx, p.ncb, (unsigned)d.BH());
-  hipLaunchKernelGGL((laplace_bwd_bcast_kernel<T, MC, DQ, DK, GSRC, RPW>), grid, dim3(64 * p.W), p.lds, st,
+  auto kern = laplace_bwd_bcast_kernel<T, MC, DQ, DK, GSRC, RPW>;
+  // M = 16 with one batch of rows per wave: one step loop, in registers that two workgroups share (bcast_paired;
+  // 64 slices of 50 rows 5.5 against 5.7 us). More rows: both loops (24 slices of 3000 rows, C = 64: 17.8
+  // against 20.5 us).
+  if constexpr (MC == 16 && bcast_paired<T, MC, DQ, DK, GSRC, RPW>())
+    if (p.rowsPerWave <= kBcRB) kern = laplace_bwd_bcast_kernel<T, MC, DQ, DK, GSRC, RPW, false>;
+  hipLaunchKernelGGL(kern, grid, dim3(64 * p.W), p.lds, st,
                      static_cast<const T*>(g), kg.src, kg.scale, static_cast<const T*>(q),
                      static_cast<const T*>(k), static_cast<T*>(dq), static_cast<T*>(dk),
                      static_cast<float*>(ws), (int)d.N, (int)d.C, p.rowsPerWave);
@@ -1884,24 +1893,33 @@ MbPlan plan_mb(const Dims& d, bool dkey) {
 // batch's missing rows too (on zero grad) and whose instructions a few rows do not pay back:
 //   up to 6 rows (fp32 grad_query, one row, M = 32: 4.6 us against 6.4 unrolled; five rows 6.1
 //   against 6.8);
-//   where three waves or more per SIMD have rows, so that issue slots count, and the missing rows
-//   cost more than the loop: 2, 3, 8 % of the rows for grad_key, grad_query, both, 50 % for both of
-//   a kernel gradient, whose loop spills (bf16 grad_query, C = 64: 2048 slices of 9 rows, M = 196, 90
-//   against 98 us; 4 of 17 rows, M = 196, 14.7 against 15.6; 256 of 130 rows, M = 17, 11.3 against
-//   12.0; fp16 kernel gradient, 64 slices of 50 rows, M = 64, 18.2 looped against 17.4).
+//   where three waves or more per SIMD have rows, so that issue slots count, and
+//   - one gradient, and the short batch is a round of its own with more than a quarter of all rounds'
+//     rows missing (bf16 grad_query: 4 of 17 rows, M = 196, 14.7 against 15.6; 256 of 130 rows, M = 17, 11.3
+//     against 12.0; M = 64, three rounds, is the faster unrolled), or
+//   - the missing rows are more than 8 % of the rows (bf16 grad_query, 2048 slices of 9 rows, M = 196,
+//     C = 64: 90 against 98 us); within two rounds 2 % for grad_key and 3 % for grad_query of 16-bit
+//     types (256 x 100 rows, M = 17: 1.016 against 1.05 of the time before the unrolled batch; in more
+//     rounds 300 x 100 rows, M = 196, take 71 us looped and 67 unrolled); 15 % for one fp32 gradient,
+//     whose loop has the slower step only (64 of 50 rows, M = 100, 17.1 looped against 15.9), 50 % for
+//     both of a kernel gradient, whose loop spills (fp16, 64 of 50 rows, M = 64, 18.2 looped against 17.4).
 // Full batches are faster unrolled at any count (fp32 grad_query, 300 slices of 64 rows, M = 64:
 // 0.9 of the loop's time). Several workgroups per slice: only the last can have a short batch.
-bool mb_row_loop(const Dims& d, const MbPlan& p, bool dq, bool dk, int gsrc) {
+bool mb_row_loop(const Dims& d, const MbPlan& p, bool f32, bool dq, bool dk, int gsrc) {
   if (p.nx > 1 || d.N < 1) return false;
-  const int64_t padded = (d.N + kMbRB - 1) / kMbRB * kMbRB;
-  const int percent = gsrc == kGradKernel ? 50 : dq && dk ? 8 : dq ? 3 : 2;
-  return d.N <= 6 || (padded / kMbRB * p.CB >= 12 && 100 * padded > (100 + percent) * d.N);
+  if (d.N <= 6) return true;
+  const int64_t batches = (d.N + kMbRB - 1) / kMbRB, rounds = (batches + p.RG - 1) / p.RG;
+  if (batches * p.CB < 12) return false;
+  const int64_t missing = batches * kMbRB - d.N;
+  if (!(dq && dk) && (batches - 1) % p.RG == 0 && 4 * missing > kMbRB * rounds) return true;
+  const int percent = gsrc == kGradKernel ? 50 : f32 && !(dq && dk) ? 15 : (dq && dk) || rounds > 2 ? 8 : dq ? 3 : 2;
+  return 100 * missing > percent * d.N;
 }
 
 template <typename T, int CB, bool DQ, bool DK, int GSRC = kGradF16>
 int launch_mb_cb(const void* g, const void* q, const void* k, void* dq, void* dk, void* ws, const Dims& d,
                  const MbPlan& p, hipStream_t st, const KernGrad& kg = {}) {
-  auto kern = mb_row_loop(d, p, DQ, DK, GSRC) ? laplace_bwd_mb_kernel<T, CB, DQ, DK, GSRC, true> : laplace_bwd_mb_kernel<T, CB, DQ, DK, GSRC>;
+  auto kern = mb_row_loop(d, p, sizeof(T) == 4, DQ, DK, GSRC) ? laplace_bwd_mb_kernel<T, CB, DQ, DK, GSRC, true> : laplace_bwd_mb_kernel<T, CB, DQ, DK, GSRC>;
   if (p.lds > 65536)
     if (int s = set_dyn_lds(reinterpret_cast<const void*>(kern), p.lds, "laplace backward")) return s;
   dim3 grid(p.nx, p.ncb, (unsigned)d.BH());

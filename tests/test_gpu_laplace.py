@@ -93,11 +93,13 @@ def test_laplace_parity(gpu, shape, dt):
 @pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("B,N,M,C", [(2, 6, 100, 64), (2, 7, 100, 64), (3, 9, 196, 40), (3, 16, 196, 64),
                                      (2, 17, 100, 64), (2, 17, 96, 64), (2, 130, 17, 70), (2, 128, 17, 64),
-                                     (2, 50, 64, 64), (2, 33, 255, 64)], ids=lambda v: str(v))
+                                     (2, 50, 64, 64), (2, 33, 255, 64), (2, 50, 16, 64),
+                                     (2, 4096, 16, 70)], ids=lambda v: str(v))
 def test_laplace_backward_short_batches(gpu, dt, B, N, M, C):
     """The column-block backward on both sides of its rule for rows in a loop: up to six rows and
     seven; short last batches where three waves per SIMD have rows and where fewer do; full batches
-    only; a last column block of one column and of 31."""
+    only; a last column block of one column and of 31. M = 16: the register-column kernel with one
+    batch of rows per wave and with more (fp32 grad_query: one step loop and two)."""
     print(f"laplace short batches {dt} B={B} N={N} M={M} C={C}", flush=True)
     q, k, g = _inputs(B, 1, N, M, C, dt, seed=1700 + N + M + C)
     out, dq, dk, dq2, dk2 = _run(gpu, q, k, g)
